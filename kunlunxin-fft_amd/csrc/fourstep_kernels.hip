@@ -16,11 +16,23 @@
 // run along the columns, so every row access is a C*8-byte contiguous run),
 // keeps them in LDS, and runs the same Stockham passes as the single-pass
 // kernel on each column.  Inverse = conjugated roots; the norm scale is applied
-// by pass 2's store.  The big twiddle W_N^e (e < N) is the product of two
-// small tables, W_N^(e mod 2^h) * W_N^(2^h * (e >> h)); pass 1 applies it in
-// registers after its last Stockham pass, as W_N^(n2*b) * (W_N^(n2*NS))^q,
-// so each thread does a few table lookups instead of two per element.
-// Stockham twiddles come from per-pass tables (rows W^k, W^2k, W^4k, W^8k).
+// by pass 2's store.
+// The twiddle W_N^(n2*k1) costs no product of its own: an N2-point FFT of
+// inputs times w^n2, w = W_N^k1, is the same FFT network with other roots
+// (its outputs are the input polynomial at w W_N2^k2 instead of W_N2^k2), so
+// pass 2 takes it into the roots of its merged butterflies (dft_dit, PassRoots)
+// and pass 1 stores plain column transforms.
+// Where the passes already move their bytes at the rate of a copy, vector
+// instructions are what is left to save: a timing-only build without butterflies and
+// twiddles ran N = 2^20, B = 64 in 345 us against 380.  Multiplying pass 1's
+// outputs by the twiddle and pass 2's inputs by pass twiddles took 3151 vector
+// instructions per thread over the two passes at 1024 points and 32 elements;
+// merged they take 2522.  N = 2^20, B = 64: 376 -> 362 us; 2^16, B = 256: 87 ->
+// 83; C2R 2^18, B = 256: 195 -> 181; R2C: 226 -> 217; 2^16, B = 32: 15.8 -> 14.3.
+// Those roots are products of a Stockham root, from a per-pass table (rows
+// W^k, W^2k, W^4k, ...) that both passes have, and of W_N^(2^t k1), t < log2
+// N2, from one row per t of N1 entries: both loads are contiguous or shared
+// across the lanes of a column group.
 #include "mfft_device.hpp"
 #include "mfft_internal.hpp"
 
@@ -141,55 +153,37 @@ __device__ __forceinline__ float2 opaque(float2 x) {
     return x;
 }
 
-// W_N^e for e < N as the product of the two small tables
-__device__ __forceinline__ float2 big_root(const float2* __restrict__ lo, const float2* __restrict__ hi,
-                                          int h, uint32_t e) {
-    return cmul(lo[e & ((1u << h) - 1)], hi[e >> h]);
-}
-
-// Pass-1 four-step twiddles of one thread, for its column n2: the outputs of
-// last-pass butterfly b = j + m*T sit at k1 = b + q*NS, so W_N^(n2*k1) =
-// W_N^(n2*b) * (W_N^(n2*NS))^q.  Holds W_N^(n2*b) per butterfly and
-// W_N^(n2*NS*2^i); the other powers are composed when applied.
-template <class C>
-struct BigTw {
-    float2 w0[C::NB_LAST];
-    float2 sp[C::LR_LAST];
-};
-
-template <class C>
-__device__ __forceinline__ void big_tw_load(BigTw<C>& f, const float2* __restrict__ lo,
-                                            const float2* __restrict__ hi, int h, uint32_t n2, int j) {
-    static_for<0, C::NB_LAST>([&](auto m) { f.w0[m.value] = big_root(lo, hi, h, n2 * (uint32_t)(j + m.value * C::T)); });
-    static_for<0, C::LR_LAST>([&](auto i) {
-        f.sp[i.value] = big_root(lo, hi, h, n2 * (uint32_t)(C::NS_LAST << i.value));
-    });
-}
-
-template <class C, int DIR, int M, int E>
-__device__ __forceinline__ void big_tw_apply(float2 (&v)[E], const BigTw<C>& f) {
-    constexpr int R = C::R_LAST;
-    if constexpr (R <= 16) {
-        float2 s[R];
-        static_for<0, C::LR_LAST>([&](auto i) { s[1 << i.value] = f.sp[i.value]; });
-        static_for<3, R>([&](auto q) {
-            constexpr int hb = high_bit(q.value);
-            if constexpr (hb != q.value) s[q.value] = cmul(s[q.value - hb], s[hb]);
-        });
-        v[M * R] = cmul_tw<DIR>(v[M * R], f.w0[M]);
-        static_for<1, R>([&](auto q) {
-            v[M * R + q.value] = cmul_tw<DIR>(v[M * R + q.value], cmul(f.w0[M], s[q.value]));
-        });
-    } else {
-        // radix 32: one factor per set bit of q (no table of R powers in registers)
-        static_for<0, R>([&](auto q) { v[M * R + q.value] = cmul_tw<DIR>(v[M * R + q.value], f.w0[M]); });
-        static_for<0, C::LR_LAST>([&](auto i) {
-            static_for<1, R>([&](auto q) {
-                if constexpr ((q.value >> i.value) & 1)
-                    v[M * R + q.value] = cmul_tw<DIR>(v[M * R + q.value], f.sp[i.value]);
-            });
+// Roots of one pass's butterfly b (dft_dit's r: r[i] = w^(2^i)).  KIND 0, a
+// plain column FFT: w = W_(NS R)^k, k = b mod NS, from the pass table tw.
+// KIND 1, the column FFT of inputs times W_N^(col n): the pass combines inputs
+// b + q L / R and carries the L / (NS R)-spaced powers that the passes before
+// it left over, so w = W_N^(col L / (NS R)) W_(NS R)^k.  col_tw: the table of
+// W_N^(2^t col), 2^log_s entries a row, at this column.
+template <class C, int KIND>
+struct PassRoots {
+    const float2* tw;
+    const float2* col_tw;  // KIND 1
+    int log_s;             // KIND 1
+    template <int p, int m, int NR>  // b = j + m T
+    __device__ __forceinline__ void load(float2 (&r)[NR], int b) const {
+        constexpr int LR = C::logr(p), LNS = C::lns(p);
+        const int k = b & ((1 << LNS) - 1);
+        static_for<0, LR>([&](auto i) {
+            float2 w = make_float2(1.0f, 0.0f);
+            if constexpr (KIND == 1) w = col_tw[(C::LOG_L - LNS - LR + i.value) << log_s];
+            if constexpr (p > 0) {
+                const float2 s = tw[sched_tw_off(C::LOG_L, C::LOG_E, p) + (i.value << LNS) + k];
+                w = KIND == 1 ? cmul(w, s) : s;
+            }
+            r[i.value] = w;
         });
     }
+};
+// Levels of a twiddled radix-2^lr DFT that take the short butterfly: as many
+// as keep the error against 64 bits at or below that of a separate product by
+// W_N^(n2*k1).  Pass 2's roots are rounded products, so it takes one less.
+constexpr int col_six(int lr, int kind) {
+    return lr >= 5 ? 3 - kind : (lr == 4 ? 2 - kind : (lr == 3 ? 1 : 0));
 }
 
 // Pass-0 operands of one column group: s = the group's first element of the
@@ -229,14 +223,13 @@ __device__ __forceinline__ void col_load(float2 (&v)[C::E], const float2* s, int
 // its operands from this thread's column in LDS; every pass but the last
 // writes its outputs back (float2 through `lds`, or, SPLIT, one component at
 // a time through the same memory as floats).  The last pass leaves its
-// outputs in registers, multiplied by the four-step twiddles for KIND 0,
-// which big() returns when the last pass starts (so they are not held in
-// registers through the earlier passes).  tw: the pass twiddle table, in
-// global memory or LDS.  With BARRIER0 the first LDS write also waits for
-// the previous group's LDS readers.
-template <class C, int DIR, int KIND, bool BARRIER0, class BigF>
-__device__ __forceinline__ void col_passes(float2 (&v)[C::E], float2* lds, const float2* tw, int c, int j,
-                                           BigF&& big) {
+// outputs in registers.  roots.load gives the roots of a pass's
+// butterflies when that pass starts; r0: those of pass 0 (KIND 1), which the
+// caller loads ahead of the operands.  With BARRIER0 the first LDS write also
+// waits for the previous group's LDS readers.
+template <class C, int DIR, int KIND, bool BARRIER0, class RootsT>
+__device__ __forceinline__ void col_passes(float2 (&v)[C::E], float2* lds, int c, int j, const float2 (&r0)[C::LOG_E],
+                                           const RootsT& roots) {
     constexpr int L = C::L, E = C::E, T = C::T, P = C::P;
     float2* lt = lds + c * C::PITCH;
     float* ltf = reinterpret_cast<float*>(lds) + c * C::PITCHF;
@@ -255,16 +248,14 @@ __device__ __forceinline__ void col_passes(float2 (&v)[C::E], float2* lds, const
                 });
             });
         }
-        BigTw<C> f;
-        if constexpr (KIND == 0 && p == P - 1) f = big();
         static_for<0, NB>([&](auto m) {
-            const int b = j + m.value * T;
-            if constexpr (NS > 1) {
-                constexpr int TW_OFF = sched_tw_off(C::LOG_L, C::LOG_E, p);
-                pass_twiddle<R, DIR, m.value * R>(v, tw + TW_OFF, NS, b & (NS - 1));
+            if constexpr (p == 0) {
+                dft_dit<R, DIR, m.value * R, KIND == 1, col_six(LR, KIND)>(v, r0);
+            } else {
+                float2 r[LR];
+                roots.template load<p, m.value>(r, j + m.value * T);
+                dft_dit<R, DIR, m.value * R, true, col_six(LR, KIND)>(v, r);
             }
-            dft<R, DIR, m.value * R, 1>(v);
-            if constexpr (KIND == 0 && p == P - 1) big_tw_apply<C, DIR, m.value>(v, f);
         });
         if constexpr (p < P - 1 && !C::SPLIT) {
             if constexpr (p > 0 || BARRIER0) __syncthreads();
@@ -420,8 +411,7 @@ __device__ __forceinline__ void col_store(const float2 (&v)[C::E], float2* d, fl
 template <int LOGL, int LOGE, int LOGC, int DIR, int KIND>
 __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_pass_kernel(
     const float2* src, float2* dst, const float2* __restrict__ tw,
-    const float2* __restrict__ tw_lo, const float2* __restrict__ tw_hi, int tw_h, int logn,
-    int log_s, float scale, int rev) {
+    const float2* __restrict__ tw_col, int logn, int log_s, float scale, int rev) {
     using C = ColCfg<LOGL, LOGE, LOGC>;
     __shared__ float2 lds[C::LDS_FLOAT2];
     const int groups = (1 << log_s) >> LOGC;  // column groups per transform
@@ -436,13 +426,11 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_pass_
     const int j = tid >> LOGC;
     const int64_t base = row << logn;
 
-    float2 v[C::E];
+    const PassRoots<C, KIND> roots{tw, tw_col + c0 + c, log_s};
+    float2 v[C::E], r0[C::LOG_E];
+    if constexpr (KIND == 1) roots.template load<0, 0>(r0, j);
     col_load<C>(v, src + base + c0, c, j, log_s);
-    col_passes<C, DIR, KIND, false>(v, lds, tw, c, j, [&] {
-        BigTw<C> f;
-        big_tw_load<C>(f, tw_lo, tw_hi, tw_h, (uint32_t)(c0 + c), j);
-        return f;
-    });
+    col_passes<C, DIR, KIND, false>(v, lds, c, j, r0, roots);
     col_store<C, KIND>(v, KIND == 0 ? dst + base + ((int64_t)c0 << LOGL) : dst + base + c0, lds, tid, c, j,
                        log_s, scale);
 }
@@ -452,8 +440,7 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_pass_
 // its CP mirror pairs per workgroup.
 template <int LOGL, int LOGE, int LOGC, int CP = 8>
 __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_r2c_pass1_kernel(
-    const float2* src, float2* dst, const float2* __restrict__ tw, const float2* __restrict__ tw_lo,
-    const float2* __restrict__ tw_hi, int tw_h, int logn, int log_s) {
+    const float2* src, float2* dst, const float2* __restrict__ tw, int logn, int log_s) {
     using C = ColCfg<LOGL, LOGE, LOGC>;
     __shared__ float2 lds[C::LDS_FLOAT2];
     const int groups = (1 << log_s) >> LOGC;
@@ -465,12 +452,9 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_r2c_p
     const int j = tid >> LOGC;
     const int64_t base = row << logn;
     float2 v[C::E];
+    const float2 r0[C::LOG_E] = {};  // pass 0 has no roots
     col_load<C>(v, src + base + c0, c, j, log_s);
-    col_passes<C, -1, 0, false>(v, lds, tw, c, j, [&] {
-        BigTw<C> f;
-        big_tw_load<C>(f, tw_lo, tw_hi, tw_h, (uint32_t)(c0 + c), j);
-        return f;
-    });
+    col_passes<C, -1, 0, false>(v, lds, c, j, r0, PassRoots<C, 0>{tw, nullptr, 0});
     col_store<C, 0, 1, false, CP>(v, dst + base + ((int64_t)c0 << LOGL), lds, tid, c, j, log_s, 1.0f);
 }
 
@@ -491,8 +475,8 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_r2c_p
 // tw_a[k1] tw_b[j] exp(-2 pi i K / (2 N2)), K = k2 - j.
 template <int LOGL, int LOGE, int LOGC>
 __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_r2c_pass2_kernel(
-    const float2* src, float2* dst, const float2* __restrict__ tw, const float2* __restrict__ tw_a,
-    const float2* __restrict__ tw_b, int logn, int log_s, float scale) {
+    const float2* src, float2* dst, const float2* __restrict__ tw, const float2* __restrict__ tw_col,
+    const float2* __restrict__ tw_a, const float2* __restrict__ tw_b, int logn, int log_s, float scale) {
     using C = ColCfg<LOGL, LOGE, LOGC>;
     static_assert(LOGC == 4 || LOGC == 5, "8 or 16 mirror pairs per workgroup");
     constexpr int CP = C::C / 2;  // mirror pairs per workgroup
@@ -507,10 +491,12 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_r2c_p
     const int c = tid & (C::C - 1);
     const int j = mirror_row_set<C::T, LOGC>(tid >> LOGC);
     const int64_t np = (int64_t)1 << logn;  // core length L = n/2
-    float2 v[E];
-    col_load<C>(v, src + (row << logn) + (g << LOGC), c, j, log_s);
-    col_passes<C, -1, 1, false>(v, lds, tw, c, j, [&] { return BigTw<C>{}; });
     const int k1 = pair_col<CP>(g, c, n1);
+    const PassRoots<C, 1> roots{tw, tw_col + k1, log_s};
+    float2 v[E], r0[C::LOG_E];
+    roots.template load<0, 0>(r0, j);
+    col_load<C>(v, src + (row << logn) + (g << LOGC), c, j, log_s);
+    col_passes<C, -1, 1, false>(v, lds, c, j, r0, roots);
     const bool col0 = g == 0 && c == 0;
     float2* xo = dst + row * (np + 1) + k1;
     // K = k2 - j of element e
@@ -555,8 +541,7 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_r2c_p
 // which are not line-aligned, so fewer lines are shared with the neighbouring
 // workgroups), turns every bin into its core input with its
 // mirror's value, then runs the column pass of the half-length inverse core
-// with its four-step twiddle and stores Z in place of the output row (the row
-// pass runs in place there).
+// and stores Z in place of the output row (the row pass runs in place there).
 // The mirror of bin (n1, n2) is (N1 - 1 - n1, N2 - n2), and thread j's rows
 // j + m T + q N1/R0 (element e = m R0 + q) have their mirrors in element
 // E - 1 - e of thread T - 1 - j, lane column c ^ CP.  Threads are laid out
@@ -571,9 +556,8 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_r2c_p
 // tw_a[n2] * tw_b[n1].
 template <int LOGL, int LOGE, int LOGC>
 __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_c2r_pass1_kernel(
-    const float2* src, float2* dst, const float2* __restrict__ tw, const float2* __restrict__ tw_lo,
-    const float2* __restrict__ tw_hi, int tw_h, const float2* __restrict__ tw_a, const float2* __restrict__ tw_b,
-    int logn, int log_s) {
+    const float2* src, float2* dst, const float2* __restrict__ tw, const float2* __restrict__ tw_a,
+    const float2* __restrict__ tw_b, int logn, int log_s) {
     using C = ColCfg<LOGL, LOGE, LOGC>;
     static_assert(LOGC == 4 || LOGC == 5, "8 or 16 mirror pairs per workgroup");
     constexpr int CP = C::C / 2;  // mirror pairs per workgroup
@@ -645,13 +629,37 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_c2r_p
             __builtin_amdgcn_sched_barrier(0);  // one element's reads at a time
         });
     }
-    col_passes<C, 1, 0, true>(v, lds, tw, c, j, [&] {
-        BigTw<C> f;
-        big_tw_load<C>(f, tw_lo, tw_hi, tw_h, (uint32_t)n2, j);
-        return f;
-    });
+    const float2 r0[C::LOG_E] = {};  // pass 0 has no roots
+    col_passes<C, 1, 0, true>(v, lds, c, j, r0, PassRoots<C, 0>{tw, nullptr, 0});
     col_store<C, 0, 2>(v, dst + (row << logn), lds, tid, c, j, log_s, 1.0f, g);
 }
+
+// The pass-2 roots of one thread (PassRoots, KIND 1) held in registers: its
+// column and its butterflies do not change from group to group.
+template <class C, int KIND>
+struct HeldRoots {
+    static constexpr int first(int p) {  // roots of the passes before p
+        int n = 0;
+        for (int q = 0; q < p; ++q) n += (C::E >> C::logr(q)) * C::logr(q);
+        return n;
+    }
+    float2 w[KIND == 1 ? first(C::P) : 1];
+    __device__ __forceinline__ void fill(const PassRoots<C, 1>& from, int j) {
+        static_for<0, C::P>([&](auto p) {
+            constexpr int LR = C::logr(p.value);
+            static_for<0, (C::E >> LR)>([&](auto m) {
+                float2 r[LR];
+                from.template load<p.value, m.value>(r, j + m.value * C::T);
+                static_for<0, LR>([&](auto i) { w[first(p.value) + m.value * LR + i.value] = r[i.value]; });
+            });
+        });
+    }
+    template <int p, int m, int NR>
+    __device__ __forceinline__ void load(float2 (&r)[NR], int) const {
+        constexpr int LR = C::logr(p);
+        static_for<0, LR>([&](auto i) { r[i.value] = opaque(w[first(p) + m * LR + i.value]); });
+    }
+};
 
 // Persistent form of the same pass: gridDim.x blocks, a multiple of the
 // column groups per transform, walk the `tiles` column groups of the launch
@@ -664,8 +672,7 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_c2r_p
 template <int LOGL, int LOGE, int LOGC, int DIR, int KIND>
 __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG), 4) void fourstep_persist_kernel(
     const float2* src, float2* dst, const float2* __restrict__ tw,
-    const float2* __restrict__ tw_lo, const float2* __restrict__ tw_hi, int tw_h, int logn,
-    int log_s, float scale, int64_t tiles, int rev) {
+    const float2* __restrict__ tw_col, int logn, int log_s, float scale, int64_t tiles, int rev) {
     using C = ColCfg<LOGL, LOGE, LOGC>;
     __shared__ float2 lds[C::LDS_FLOAT2];
     __shared__ float2 lds_tw[C::TW_SIZE > 0 ? C::TW_SIZE : 1];
@@ -680,9 +687,11 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG), 4) void fourstep_pe
     const int64_t last_row = (tiles >> log_groups) - 1;
     auto row_of = [&](int64_t t) { return (KIND == 1 && rev) ? last_row - (t >> log_groups) : (t >> log_groups); };
 
-    for (int i = tid; i < C::TW_SIZE; i += C::WG) lds_tw[i] = tw[i];
-    BigTw<C> f;
-    if constexpr (KIND == 0) big_tw_load<C>(f, tw_lo, tw_hi, tw_h, (uint32_t)(c0 + c), j);
+    if constexpr (KIND == 0) {
+        for (int i = tid; i < C::TW_SIZE; i += C::WG) lds_tw[i] = tw[i];
+    }
+    HeldRoots<C, KIND> held;
+    if constexpr (KIND == 1) held.fill(PassRoots<C, 1>{tw, tw_col + c0 + c, log_s}, j);
     float2 v[C::E];
     col_load<C>(v, src + (row_of(t0) << logn) + c0, c, j, log_s);
     __syncthreads();  // lds_tw complete
@@ -693,12 +702,14 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG), 4) void fourstep_pe
     // across the loop (next to the prefetched group) would take.
     auto process = [&](int64_t t) {
         const int jl = opaque(j), cl = opaque(c), tl = opaque(tid);
-        col_passes<C, DIR, KIND, true>(v, lds, lds_tw, cl, jl, [&] {
-            BigTw<C> fl;
-            static_for<0, C::NB_LAST>([&](auto m) { fl.w0[m.value] = opaque(f.w0[m.value]); });
-            static_for<0, C::LR_LAST>([&](auto i) { fl.sp[i.value] = opaque(f.sp[i.value]); });
-            return fl;
-        });
+        if constexpr (KIND == 1) {
+            float2 r0[C::LOG_E];
+            held.template load<0, 0>(r0, jl);
+            col_passes<C, DIR, 1, true>(v, lds, cl, jl, r0, held);
+        } else {
+            const float2 r0[C::LOG_E] = {};  // pass 0 has no roots
+            col_passes<C, DIR, 0, true>(v, lds, cl, jl, r0, PassRoots<C, 0>{lds_tw, nullptr, 0});
+        }
         const int64_t base = row_of(t) << logn;
         col_store<C, KIND>(v, dst + opaque_uniform(KIND == 0 ? base + ((int64_t)c0 << LOGL) : base + c0), lds, tl, cl,
                            jl, log_s, scale);
@@ -769,8 +780,7 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG), 4) void fourstep_pe
 template <int LL1, int LE1, int LC1, int LL2, int LE2, int LC2, int DIR>
 __global__ __launch_bounds__((ColCfg<LL1, LE1, LC1>::WG)) void fourstep_fused_kernel(
     const float2* src, float2* dst, float2* ring, const float2* __restrict__ tw1, const float2* __restrict__ tw2,
-    const float2* __restrict__ tw_lo, const float2* __restrict__ tw_hi, int tw_h, float scale, int rows,
-    int nslot, int lag, int nring, int per_take, int* sync, int* overrun, long long wait_ticks) {
+    const float2* __restrict__ tw_col, float scale, int rows, int nslot, int lag, int nring, int per_take, int* sync, int* overrun, long long wait_ticks) {
     using A = ColCfg<LL1, LE1, LC1>;
     using B = ColCfg<LL2, LE2, LC2>;
     static_assert(A::WG == B::WG, "both passes run with the same block size");
@@ -848,11 +858,8 @@ __global__ __launch_bounds__((ColCfg<LL1, LE1, LC1>::WG)) void fourstep_fused_ke
             const int c = tl & (A::C - 1), j = tl >> LC1, c0 = g << LC1;
             float2 v[A::E];
             col_load<A>(v, src + ((int64_t)t << LOGN) + c0, c, j, LL2);
-            col_passes<A, DIR, 0, true>(v, lds, tw1, c, j, [&] {
-                BigTw<A> f;
-                big_tw_load<A>(f, tw_lo, tw_hi, tw_h, (uint32_t)(c0 + c), j);
-                return f;
-            });
+            const float2 r0[A::LOG_E] = {};  // pass 0 has no roots
+            col_passes<A, DIR, 0, true>(v, lds, c, j, r0, PassRoots<A, 0>{tw1, nullptr, 0});
             // the ring slot is free once every pass-2 group of k - R has read it
             int ok = 1;
             if (k >= nring) {
@@ -874,9 +881,11 @@ __global__ __launch_bounds__((ColCfg<LL1, LE1, LC1>::WG)) void fourstep_fused_ke
             __syncthreads();
             const int failed = __builtin_amdgcn_readfirstlane(fail_s);
             const int c = tl & (B::C - 1), j = tl >> LC2, c0 = g << LC2;
-            float2 v[B::E];
+            const PassRoots<B, 1> roots{tw2, tw_col + c0 + c, LL1};
+            float2 v[B::E], r0[B::LOG_E];
+            roots.template load<0, 0>(r0, j);
             col_load<B, true>(v, zr + c0, c, j, LL1);
-            col_passes<B, DIR, 1, true>(v, lds, tw2, c, j, [&] { return BigTw<B>{}; });
+            col_passes<B, DIR, 1, true>(v, lds, c, j, r0, roots);
             // a failed launch writes NaN, not a transform of partial data
             col_store<B, 1, 0, true>(v, dst + ((int64_t)t << LOGN) + c0, lds, tl, c, j, LL1,
                                      failed ? __builtin_nanf("") : scale);
@@ -921,7 +930,7 @@ hipError_t launch_pass_narrow(const float2* src, float2* dst, const mfft_plan* p
     const int64_t tiles = rows * (((int64_t)1 << log_s) >> LOGC);
     if (!launch_fits(tiles, C::WG)) return hipErrorInvalidConfiguration;
     fourstep_pass_kernel<LOGL, LOGE, LOGC, DIR, KIND><<<(unsigned)tiles, C::WG, 0, stream>>>(
-        src, dst, KIND == 0 ? p->tw_n1 : p->tw_n2, p->tw_lo, p->tw_hi, p->tw_h, logn, log_s, scale, p->pass2_rev);
+        src, dst, KIND == 0 ? p->tw_n1 : p->tw_n2, p->tw_col, logn, log_s, scale, p->pass2_rev);
     mark(stream);
     return hipGetLastError();
 }
@@ -947,10 +956,10 @@ hipError_t launch_pass(const float2* src, float2* dst, const mfft_plan* p, int64
         if (g < unit) g = unit;
         if (g > tiles) g = tiles;
         fourstep_persist_kernel<LOGL, LOGE, LOGC, DIR, KIND><<<(unsigned)g, C::WG, 0, stream>>>(
-            src, dst, tw, p->tw_lo, p->tw_hi, p->tw_h, logn, log_s, scale, tiles, p->pass2_rev);
+            src, dst, tw, p->tw_col, logn, log_s, scale, tiles, p->pass2_rev);
     } else {
         fourstep_pass_kernel<LOGL, LOGE, LOGC, DIR, KIND><<<(unsigned)tiles, C::WG, 0, stream>>>(
-            src, dst, tw, p->tw_lo, p->tw_hi, p->tw_h, logn, log_s, scale, p->pass2_rev);
+            src, dst, tw, p->tw_col, logn, log_s, scale, p->pass2_rev);
     }
     mark(stream);
     return hipGetLastError();
@@ -976,34 +985,34 @@ hipError_t launch_real_pass(const float2* src, float2* dst, const mfft_plan* p, 
     if constexpr (KIND == 0) {
         if (LOGL >= 5 && log_s <= 9)
             fourstep_r2c_pass1_kernel<LOGL, LOGE, LOGC, 16><<<(unsigned)tiles, C::WG, 0, stream>>>(
-                src, dst, p->tw_n1, p->tw_lo, p->tw_hi, p->tw_h, logn, log_s);
+                src, dst, p->tw_n1, logn, log_s);
         else
             fourstep_r2c_pass1_kernel<LOGL, LOGE, LOGC><<<(unsigned)tiles, C::WG, 0, stream>>>(
-                src, dst, p->tw_n1, p->tw_lo, p->tw_hi, p->tw_h, logn, log_s);
+                src, dst, p->tw_n1, logn, log_s);
     } else if constexpr (KIND == 1) {
         bool pairs16 = false;
         if constexpr (LOGL <= 9) {
             if (log_s >= 5) {
                 pairs16 = true;
                 fourstep_r2c_pass2_kernel<LOGL, LOGE, 5><<<(unsigned)(tiles >> 1), C5::WG, 0, stream>>>(
-                    src, dst, p->tw_n2, p->tw_ra, p->tw_rb, logn, log_s, scale);
+                    src, dst, p->tw_n2, p->tw_col, p->tw_ra, p->tw_rb, logn, log_s, scale);
             }
         }
         if (!pairs16)
             fourstep_r2c_pass2_kernel<LOGL, LOGE, LOGC><<<(unsigned)tiles, C::WG, 0, stream>>>(
-                src, dst, p->tw_n2, p->tw_ra, p->tw_rb, logn, log_s, scale);
+                src, dst, p->tw_n2, p->tw_col, p->tw_ra, p->tw_rb, logn, log_s, scale);
     } else {
         bool pairs16 = false;
         if constexpr (LOGL <= 9) {
             if (log_s >= 5) {
                 pairs16 = true;
                 fourstep_c2r_pass1_kernel<LOGL, LOGE, 5><<<(unsigned)(tiles >> 1), C5::WG, 0, stream>>>(
-                    src, dst, p->tw_n1, p->tw_lo, p->tw_hi, p->tw_h, p->tw_ra, p->tw_rb, logn, log_s);
+                    src, dst, p->tw_n1, p->tw_ra, p->tw_rb, logn, log_s);
             }
         }
         if (!pairs16)
             fourstep_c2r_pass1_kernel<LOGL, LOGE, LOGC><<<(unsigned)tiles, C::WG, 0, stream>>>(
-                src, dst, p->tw_n1, p->tw_lo, p->tw_hi, p->tw_h, p->tw_ra, p->tw_rb, logn, log_s);
+                src, dst, p->tw_n1, p->tw_ra, p->tw_rb, logn, log_s);
     }
     mark(stream);
     return hipGetLastError();
@@ -1067,7 +1076,7 @@ hipError_t launch_fused_one(const float2* src, float2* dst, char* fws, const mff
     // grid, lag, ring and take were fixed at plan creation (one resident
     // wave of blocks, a multiple of the XCD count)
     fourstep_fused_kernel<L1, E1, C1, L2, E2, C2, DIR><<<p->fused_grid, A::WG, 0, stream>>>(
-        src, dst, ring, p->tw_n1, p->tw_n2, p->tw_lo, p->tw_hi, p->tw_h, scale, (int)rows, p->num_xcc,
+        src, dst, ring, p->tw_n1, p->tw_n2, p->tw_col, scale, (int)rows, p->num_xcc,
         p->fused_lag, p->fused_ring, p->fused_take, sync, p->overrun, (long long)kFusedWaitMs * p->clock_khz);
     mark(stream);
     return hipGetLastError();

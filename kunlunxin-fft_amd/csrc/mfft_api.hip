@@ -102,6 +102,16 @@ std::vector<float2> pass_table(int logl, int le, bool rf = false) {
     return t;
 }
 
+// The four-step twiddles W_n^(2^t k1), row t < log2n2 holding k1 < n1.  The
+// entry of an even k1 is the next row's at k1 / 2; only odd ones are computed.
+std::vector<float2> column_table(int64_t n, int64_t n1, int log2n2) {
+    std::vector<float2> t((size_t)(log2n2 * n1));
+    for (int r = log2n2 - 1; r >= 0; --r)
+        for (int64_t k = 0; k < n1; ++k)
+            t[(size_t)(r * n1 + k)] = (k & 1) || r == log2n2 - 1 ? root(n, k << r) : t[(size_t)((r + 1) * n1 + k / 2)];
+    return t;
+}
+
 // Plan uploads go through one private non-blocking stream per device, and
 // plan creation waits for that stream alone: a plan created while other
 // streams run kernels neither waits for them nor stalls them (a plain
@@ -140,8 +150,8 @@ int upload(float2** dptr, const std::vector<float2>& h, int64_t* bytes, hipStrea
 }
 
 void release(mfft_plan* p) {
-    float2** bufs[] = {&p->tw, &p->tw_n1, &p->tw_n2, &p->tw_lo,  &p->tw_hi,
-                       &p->tw_real, &p->tw_ra, &p->tw_rb, &p->ws_a, &p->ws_b};
+    float2** bufs[] = {&p->tw,      &p->tw_n1, &p->tw_n2, &p->tw_col, &p->tw_real,
+                       &p->tw_ra,   &p->tw_rb, &p->ws_a,  &p->ws_b};
     for (float2** b : bufs) {
         if (*b) (void)hipFree(*b);
         *b = nullptr;
@@ -618,13 +628,10 @@ int mfft_plan_create_ex(mfft_plan** out, int64_t n, int64_t batch, int transform
     };
     host.reserve(7);
     if (rc == MFFT_OK && flow == MFFT_FLOW_FOUR_STEP) {
-        const int lc = logc;
         const int l1 = mfft::ilog2((int)n1), l2 = mfft::ilog2((int)n2);
-        p->tw_h = (lc + 1) / 2;
-        if (rc == MFFT_OK) rc = put(&p->tw_n1, pass_table(l1, mfft::fourstep_col_loge(l1, schedule)));
+        rc = put(&p->tw_n1, pass_table(l1, mfft::fourstep_col_loge(l1, schedule)));
         if (rc == MFFT_OK) rc = put(&p->tw_n2, pass_table(l2, mfft::fourstep_col_loge(l2, schedule)));
-        if (rc == MFFT_OK) rc = put(&p->tw_lo, roots(core_n, (int64_t)1 << p->tw_h, 1));
-        if (rc == MFFT_OK) rc = put(&p->tw_hi, roots(core_n, core_n >> p->tw_h, (int64_t)1 << p->tw_h));
+        if (rc == MFFT_OK) rc = put(&p->tw_col, column_table(core_n, n1, l2));
     } else if (rc == MFFT_OK && flow == MFFT_FLOW_LDS_FUSED) {
         const int le = mfft::sched_le(logc, mfft::ilog2(elems));
         rc = put(&p->tw, pass_table(logc, le, mfft::lds_remainder_first(logc, le, p->r2c_fused)));

@@ -139,6 +139,84 @@ __device__ __forceinline__ void dft(float2 (&v)[E]) {
     }
 }
 
+// ---- radix-R DFT of twiddled inputs, the twiddles merged into its butterflies --
+// With input twiddles w^q the outputs are the values of sum_q v_q z^q at
+// z = w exp(DIR 2 pi i k / R), and decimation in time evaluates them with
+// butterflies a +- (w^(R/2^l) exp(DIR 2 pi i m / 2^l)) b, m < 2^(l-1), at
+// level l = 1 .. log2 R: the input twiddle only turns every butterfly's root,
+// and costs no product of its own.  Level l needs one loaded root w^(R/2^l)
+// and its products with the compile-time roots m < 2^(l-2); the other half
+// differs by a factor -+i, which a swap of operands applies.
+//
+// A butterfly is four FMAs for a + w b and four more for a - w b, or two:
+// 2 a - (a + w b), which also carries the first result's rounding.  The
+// short form is taken in the first SIX levels of a twiddled DFT.  Against
+// products of the inputs by w^q and a decimation-in-frequency network (272
+// operations at R = 16, 776 at R = 32, where only the log2 R loaded roots fit
+// the registers), this takes 240 and 620 with half the levels short, and its
+// error against 64 bits is 0-4% smaller; with every level short (208, 524) it
+// would be 3-6% larger (single-pass transforms of 2^8 .. 2^15 points).
+template <int DIR, bool ROT, bool SIX_OPS>
+__device__ __forceinline__ void butterfly(float2& a, float2& b, float wx, float wy) {
+    const float q = DIR < 0 ? wy : -wy;
+    // w b = (xx b.x + xy b.y, yx b.x + yy b.y), times DIR i with ROT
+    const float xx = !ROT ? wx : (DIR < 0 ? q : -q), xy = !ROT ? -q : (DIR < 0 ? wx : -wx);
+    const float yx = !ROT ? q : (DIR < 0 ? -wx : wx), yy = !ROT ? wx : (DIR < 0 ? q : -q);
+    const float sx = fmaf(xy, b.y, fmaf(xx, b.x, a.x));
+    const float sy = fmaf(yy, b.y, fmaf(yx, b.x, a.y));
+    if constexpr (SIX_OPS) {
+        b = make_float2(fmaf(2.0f, a.x, -sx), fmaf(2.0f, a.y, -sy));
+    } else {
+        b = make_float2(fmaf(-xy, b.y, fmaf(-xx, b.x, a.x)), fmaf(-yy, b.y, fmaf(-yx, b.x, a.y)));
+    }
+    a = make_float2(sx, sy);
+}
+// the same for w = 1 (times DIR i with ROT)
+template <int DIR, bool ROT>
+__device__ __forceinline__ void butterfly1(float2& a, float2& b) {
+    const float2 t = rot<4, ROT ? 1 : 0, DIR>(b);
+    b = csub(a, t);
+    a = cadd(a, t);
+}
+
+// v[OFF + q], q in [0, R): natural order in and out.  r[i] = w^(2^i) as
+// forward-table roots (DIR = +1 takes their conjugates); TW = false: w = 1,
+// r is not read.
+template <int R, int DIR, int OFF, bool TW, int SIX, int E, int NR>
+__device__ __forceinline__ void dft_dit(float2 (&v)[E], const float2 (&r)[NR]) {
+    static_assert(R >= 1 && (R & (R - 1)) == 0, "radix must be a power of two");
+    constexpr int LOGR = ilog2(R);
+    static_assert(!TW || NR >= LOGR, "one root per level");
+    if constexpr (R > 1) {
+        static_for<0, LOGR>([&](auto lv) {
+            constexpr int l = lv.value + 1;
+            constexpr int h = R >> l;                        // butterflies per root
+            constexpr int roots = l >= 2 ? 1 << (l - 2) : 1;  // distinct roots, up to -+i
+            static_for<0, roots>([&](auto mm) {
+                constexpr int m = mm.value;
+                // level l has combined the inputs of every residue mod h; block
+                // brev(m') holds the values at roots of index m'
+                auto block = [&](auto mk, auto rotated, float2 w) {
+                    constexpr int i0 = OFF + brev_bits(mk.value, l - 1) * 2 * h;
+                    static_for<0, h>([&](auto q) {
+                        if constexpr (!TW && m == 0)
+                            butterfly1<DIR, rotated.value>(v[i0 + q.value], v[i0 + q.value + h]);
+                        else
+                            butterfly<DIR, rotated.value, TW && (l <= SIX)>(v[i0 + q.value], v[i0 + q.value + h], w.x,
+                                                                            w.y);
+                    });
+                };
+                const float2 w = rot<(1 << l), m, -1>(TW ? r[TW ? LOGR - l : 0] : make_float2(1.0f, 0.0f));
+                block(ic<m>{}, std::false_type{}, w);
+                if constexpr (l >= 2) block(ic<m + roots>{}, std::true_type{}, w);
+            });
+        });
+        float2 t[R];
+        static_for<0, R>([&](auto q) { t[q.value] = v[OFF + brev_bits(q.value, LOGR)]; });
+        static_for<0, R>([&](auto q) { v[OFF + q.value] = t[q.value]; });
+    }
+}
+
 // ---- Stockham schedule shared by the host (table builder) and the kernels --
 // A transform of length 2^logl with up to 2^loge elements per thread runs P
 // passes; pass p has radix 2^logr(p) and accumulated span NS = 2^lns(p), the

@@ -37,9 +37,7 @@ struct mfft_plan {
     float2* tw = nullptr;       // stage flows: W_core^m, m in [0, core_n); LDS flow: pass table
     float2* tw_n1 = nullptr;    // four-step pass-1 Stockham pass table (length n1)
     float2* tw_n2 = nullptr;    // four-step pass-2 Stockham pass table (length n2)
-    float2* tw_lo = nullptr;    // W_core^m, m < 2^h             (four-step twiddle, low digit)
-    float2* tw_hi = nullptr;    // W_core^(m*2^h)                (four-step twiddle, high digit)
-    int tw_h = 0;
+    float2* tw_col = nullptr;   // W_core^(2^t k1): row t < log2 n2 of n1 entries (four-step twiddle)
     float2* tw_real = nullptr;  // exp(-2*pi*i*k/n), k in [0, n/2]  (r2c stitch / c2r pre)
     float2* tw_ra = nullptr;    // real four-step: r2c W_n^k1 (k1 < n1); c2r W_n^n2 (n2 < n2)
     float2* tw_rb = nullptr;    // real four-step: r2c W_n^(n1 k2) (k2 <= n2); c2r W_n^(n2 n1) (n1 < n1)

@@ -1,0 +1,61 @@
+"""Merged-twiddle butterflies: every radix, remainder radix and number of
+passes that a transform is cut into, against 64-bit numpy.
+
+The bound is on the rounding of the network itself.  A radix-2 level writes
+each value after two roundings of at most half an ulp (three where the second
+output is derived from the first), whose errors, u = 2^-24, have a variance of
+u^2/3 relative to the value; with the rounding of the roots a level adds less
+than u^2, so log2 N levels stay below u sqrt(log2 N) in the 2-norm.  A wrong
+or misplaced root gives an error of order one.
+"""
+import math
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+
+def _run(pkg, gpu, n, batch, direction, executed, params, seed):
+    import torch
+
+    rng = np.random.default_rng(seed)
+    x = (rng.standard_normal((batch, n)) + 1j * rng.standard_normal((batch, n))).astype(np.complex64)
+    plan = pkg.ExecutionPlan(n=n, batch=batch, direction="dit", precision="fp32", selection_source="table",
+                             reason="test", fallback=False, executed=executed, block=None, params=params,
+                             transform_direction=direction, norm="ortho")
+    y = pkg.execute_fft_plan(plan, torch.from_numpy(x).to(gpu)).cpu().numpy()
+    e = (np.fft.fft if direction == "forward" else np.fft.ifft)(x.astype(np.complex128), norm="ortho")
+    return float(np.linalg.norm(y - e) / np.linalg.norm(e))
+
+
+@pytest.mark.parametrize("direction", ["forward", "inverse"])
+@pytest.mark.parametrize("schedule", [0, 1, 3])
+@pytest.mark.parametrize("l1,l2", [(4, 4), (5, 4), (4, 6), (6, 5), (7, 6), (8, 7), (7, 9), (9, 8), (10, 8), (10, 10)])
+def test_four_step_split(pkg, gpu, l1, l2, schedule, direction):
+    """Pass 2's roots carry W_N^(n2 k1): every pass length 16..1024 on either
+    side, so every radix 2..32 as first, middle and remainder pass."""
+    n = 1 << (l1 + l2)
+    err = _run(pkg, gpu, n, 3, direction, "fft_four_step_batch", {"n1": 1 << l1, "schedule": schedule},
+               1000 * l1 + l2)
+    assert err <= U * math.sqrt(l1 + l2), err
+
+
+@pytest.mark.parametrize("l1,l2", [(4, 4), (5, 6), (7, 5), (8, 9), (10, 9)])
+def test_four_step_real(pkg, gpu, l1, l2):
+    """The real epilogues' row passes take the same roots at permuted (R2C)
+    and mirrored columns: forward and back returns the samples."""
+    import torch
+
+    n = 2 << (l1 + l2)
+    x = np.random.default_rng(n).standard_normal((3, n)).astype(np.float32)
+    common = dict(n=n, batch=3, direction="dit", precision="fp32", selection_source="table", reason="test",
+                  fallback=False, executed="fft_four_step_batch", block=None, params={"n1": 1 << l1}, norm="ortho")
+    spec = pkg.execute_fft_plan(pkg.ExecutionPlan(transform_type="r2c", **common), torch.from_numpy(x).to(gpu))
+    e = np.fft.rfft(x.astype(np.float64), norm="ortho")
+    levels = l1 + l2 + 2  # the core's, the stitch and the rounding of its roots
+    assert np.linalg.norm(spec.cpu().numpy() - e) <= U * math.sqrt(levels) * np.linalg.norm(e)
+    back = pkg.execute_fft_plan(pkg.ExecutionPlan(transform_type="c2r", transform_direction="inverse", **common), spec)
+    assert np.linalg.norm(back.cpu().numpy() - x) <= U * math.sqrt(2 * levels) * np.linalg.norm(x)
