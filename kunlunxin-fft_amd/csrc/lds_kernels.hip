@@ -91,6 +91,14 @@ struct LdsCfg {
     // themselves).
     static constexpr bool PAIR =
         LE >= 3 && T >= 64 && (MODE == 2 || (MODE == 1 && sched_logr(LOGL, LE, P - 1, RF) == LE));
+    // Pass twiddles merged into the butterflies (dft_dit, one level short) with
+    // 32 elements per thread: 10-15% fewer vector instructions (2^13: 1939 ->
+    // 1642, 2^15: 2324 -> 2100), N = 2^13 of 256 MiB 90 -> 87 us, 2^14 97 -> 95,
+    // 2^14, B = 256 20 -> 19.2, R2C 2^16 125 -> 122.  Up to 16 elements the
+    // products cost little more (272 operations a pass against 256) and both
+    // forms run alike (N = 4096: 82 us); at 1024 points the merged form spills
+    // (81 -> 95 us).
+    static constexpr bool MERGED = LE == 5 && LOGL >= 11;
     static constexpr int logr(int p) { return sched_logr(LOGL, LE, p, RF); }
     static constexpr int lns(int p) { return sched_lns_rf(LOGL, LE, p, RF); }
 };
@@ -142,6 +150,10 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
                   "the staged form is for transforms of fewer than 16 threads");
     // rows of L + 1 bins (R2C output, C2R input) of the staged form, flat in LDS
     static_assert(!STAGED || C::TPB * (L + 1) <= (C::LDS_FLOATS / 2), "staged bin rows exceed the LDS rows");
+    // C2C loads with a select each: at 2^15 points, one 16-wave block per CU,
+    // its exec mask spaces the 32 loads of a thread out (a batch of 1000: 107
+    // us, 109 back to back); the 32-element 1024-point kernel spills without.
+    constexpr bool SELECT = MODE == 0 && C::LE == 5 && (LOGL == 10 || LOGL == 15);
     constexpr bool NEED_LDS = (P > 1) || (MODE == 1) || STAGED;
     // write-through output stores (store_out) for C2C up to 2^13 points,
     // where every store instruction writes whole 128-byte lines: the staged
@@ -175,7 +187,10 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
     const int tl = tid / T;
     const int j = C::PAIR ? pair_j<T>(tid & (T - 1)) : tid & (T - 1);
     const int64_t row = (int64_t)blockIdx.x * C::TPB + tl;
-    const bool active = row < rows;
+    const bool active = C::TPB == 1 || row < rows;  // one transform per block: the grid is the batch
+    // the threads of rows past the batch (last block) load its last row again
+    // and store nothing: loads without a select run without exec masks
+    const int64_t lrow = active ? row : rows - 1;
     float2* lt = lds + (NEED_LDS ? tl * C::PITCH : 0);
     float* ltf = ldsf + (NEED_LDS ? tl * C::PITCH : 0);
 
@@ -218,12 +233,10 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             // j = 0 reads is still the bin: v[E-s] belongs to a later pair,
             // and v[s+1], already turned, was kept in `prev`.
             static_assert(R0 == E && NB0 == 1, "lane pairing needs a full radix first pass");
-            const float2* xb = (const float2*)src_v + row * (L + 1);
-            static_for<0, E>([&](auto q) {
-                v[q.value] = active ? load_nt(xb + j + q.value * T) : make_float2(0.0f, 0.0f);
-            });
+            const float2* xb = (const float2*)src_v + lrow * (L + 1);
+            static_for<0, E>([&](auto q) { v[q.value] = load_nt(xb + j + q.value * T); });
             const bool jz = j == 0, jh = j == T / 2;
-            const float2 xny = (active && jz) ? load_nt(xb + L) : make_float2(0.0f, 0.0f);
+            const float2 xny = jz ? load_nt(xb + L) : make_float2(0.0f, 0.0f);
             // exp(-2 pi i (j + T*s) / 2L) = tw_real[j] * exp(-2 pi i s / 2E):
             // one table load and compile-time rotations
             const float2 tj = tw_real[j];
@@ -260,14 +273,14 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             // floats): real parts first, kept in px, then imaginary parts,
             // on which the pre-twiddle is applied.  Bin L, the partner of
             // bin 0, is loaded by thread 0, which holds bin 0.
-            const float2* xb = (const float2*)src_v + row * (L + 1);
+            const float2* xb = (const float2*)src_v + lrow * (L + 1);
             static_for<0, NB0>([&](auto m) {
                 static_for<0, R0>([&](auto q) {
                     const int i = j + m.value * T + q.value * (L / R0);
-                    v[m.value * R0 + q.value] = active ? load_nt(xb + i) : make_float2(0.0f, 0.0f);
+                    v[m.value * R0 + q.value] = load_nt(xb + i);
                 });
             });
-            const float2 xny = (active && j == 0) ? load_nt(xb + L) : make_float2(0.0f, 0.0f);
+            const float2 xny = j == 0 ? load_nt(xb + L) : make_float2(0.0f, 0.0f);
             const int pjf = padf<C::FSH>(j);
             float px[E];
             static_for<0, 2>([&](auto comp) {
@@ -305,21 +318,17 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             // transform per 32 lanes (no lane pairing; the partner values
             // would not fit the register budget): both bins straight from
             // global memory
-            const float2* xb = (const float2*)src_v + row * (L + 1);
+            const float2* xb = (const float2*)src_v + lrow * (L + 1);
             static_for<0, NB0>([&](auto m) {
                 static_for<0, R0>([&](auto q) {
                     const int i = j + m.value * T + q.value * (L / R0);
-                    float2 z = make_float2(0.0f, 0.0f);
-                    if (active) {
-                        float2 xk = xb[i];
-                        float2 xj = xb[L - i];
-                        if (i == 0) {
-                            xk.y = 0.0f;
-                            xj.y = 0.0f;
-                        }
-                        z = c2r_pre_bin(xk, xj, tw_real[i]);
+                    float2 xk = xb[i];
+                    float2 xj = xb[L - i];
+                    if (i == 0) {
+                        xk.y = 0.0f;
+                        xj.y = 0.0f;
                     }
-                    v[m.value * R0 + q.value] = z;
+                    v[m.value * R0 + q.value] = c2r_pre_bin(xk, xj, tw_real[i]);
                 });
             });
         } else if constexpr (STAGED) {
@@ -342,11 +351,13 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
         } else {
             // non-temporal: every input element is read exactly once, and
             // keeping it out of L2 and the MALL measured 5-10% faster
-            const float2* src = (const float2*)src_v + row * L;
+            const float2* src = (const float2*)src_v + lrow * L;
             static_for<0, NB0>([&](auto m) {
                 static_for<0, R0>([&](auto q) {
                     const int i = j + m.value * T + q.value * (L / R0);
-                    v[m.value * R0 + q.value] = active ? load_nt(src + i) : make_float2(0.0f, 0.0f);
+                    float2& x = v[m.value * R0 + q.value];
+                    if constexpr (SELECT) x = row < rows ? load_nt(src + i) : make_float2(0.0f, 0.0f);
+                    else x = load_nt(src + i);
                 });
             });
         }
@@ -369,12 +380,16 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             });
         }
         static_for<0, NB>([&](auto m) {
-            if constexpr (NS > 1) {
-                const int b = j + m.value * T;
-                constexpr int TW_OFF = sched_tw_off(LOGL, C::LE, p, C::RF);
-                pass_twiddle<R, DIR, m.value * R, (C::WG == 1024 && E == 32)>(v, tw + TW_OFF, NS, b & (NS - 1));
+            constexpr int TW_OFF = NS > 1 ? sched_tw_off(LOGL, C::LE, p, C::RF) : 0;
+            const int k = (j + m.value * T) & (NS - 1);
+            if constexpr (C::MERGED) {
+                float2 r[LR > 0 ? LR : 1];
+                if constexpr (NS > 1) pass_roots<LR, C::WG == 1024>(r, tw + TW_OFF, NS, k);
+                dft_dit<R, DIR, m.value * R, (NS > 1), (LR >= 3 ? 1 : 0)>(v, r);
+            } else {
+                if constexpr (NS > 1) pass_twiddle<R, DIR, m.value * R>(v, tw + TW_OFF, NS, k);
+                dft<R, DIR, m.value * R, 1>(v);
             }
-            dft<R, DIR, m.value * R, 1>(v);
         });
         if constexpr ((p < P - 1 || (MODE == 1 && !C::PAIR)) && !C::SPLIT) {
             // every thread has read this pass's inputs (pass 0 of c2r: the partner bins)

@@ -149,13 +149,14 @@ __device__ __forceinline__ void dft(float2 (&v)[E]) {
 // differs by a factor -+i, which a swap of operands applies.
 //
 // A butterfly is four FMAs for a + w b and four more for a - w b, or two:
-// 2 a - (a + w b), which also carries the first result's rounding.  The
-// short form is taken in the first SIX levels of a twiddled DFT.  Against
-// products of the inputs by w^q and a decimation-in-frequency network (272
-// operations at R = 16, 776 at R = 32, where only the log2 R loaded roots fit
-// the registers), this takes 240 and 620 with half the levels short, and its
-// error against 64 bits is 0-4% smaller; with every level short (208, 524) it
-// would be 3-6% larger (single-pass transforms of 2^8 .. 2^15 points).
+// 2 a - (a + w b), which also carries the first result's rounding.  This
+// short form is taken in the first SIX levels of a twiddled DFT.  Products of
+// the inputs by w^q and then a decimation-in-frequency network take 272
+// operations at R = 16 and 776 at R = 32 (only the log2 R loaded roots fit the
+// registers beside 32 values); merged it is 256 and 652 with one level short,
+// with an error against 64 bits 0-5% smaller.  With every level short (208
+// and 524) the error would be 3-6% larger, and with the product t = w b and
+// a +- t for the long form 0-2%.
 template <int DIR, bool ROT, bool SIX_OPS>
 __device__ __forceinline__ void butterfly(float2& a, float2& b, float wx, float wy) {
     const float q = DIR < 0 ? wy : -wy;
@@ -321,25 +322,32 @@ __device__ __forceinline__ int64_t opaque_uniform(int64_t x) {
     return x;
 }
 
-// Multiply v[OFF + q] (q = 1..R-1) by W^(q*k) of a pass whose table rows
-// `tp[i*NS + k]` hold W^(2^i * k): loads the log2(R) power-of-two roots
-// (coalesced across lanes) and composes the rest, w_q = w_(q - hb) * w_hb,
-// one complex product each.
-// Radix 32 instead multiplies v[q] by w_(2^i) for every set bit i of q, so
-// only log2(R) roots are live (the composed form would hold R of them).
+// The roots r[i] = W^(2^i * k) of a pass's butterfly (dft_dit) from its table
+// rows `tp[i*NS + k]`: LR loads, coalesced across lanes.
 // SROW: address each table row as a scalar base plus the lane's 32-bit
 // offset.  Otherwise the compiler forms a 64-bit per-lane pointer per row
 // (row offsets beyond the load's immediate range), which costs the 16-wave
 // 32768-point kernels, at their 128-VGPR budget, a spilled register; where
 // registers are not that scarce the default form schedules better (measured
 // 1-3% faster at 2^10-2^17).
-template <int R, int DIR, int OFF, bool SROW = false, int E>
+template <int LR, bool SROW, int NR>
+__device__ __forceinline__ void pass_roots(float2 (&r)[NR], const float2* __restrict__ tp, int ns, int k) {
+    static_for<0, LR>([&](auto i) {
+        if constexpr (SROW) r[i.value] = *byte_off(tp + opaque_uniform((int64_t)i.value * ns), (uint32_t)k * 8u);
+        else r[i.value] = tp[i.value * ns + k];
+    });
+}
+
+// Multiply v[OFF + q] (q = 1..R-1) by W^(q*k) of a pass whose table rows
+// `tp[i*NS + k]` hold W^(2^i * k): loads the log2(R) power-of-two roots
+// (coalesced across lanes) and composes the rest, w_q = w_(q - hb) * w_hb,
+// one complex product each.
+// Radix 32 instead multiplies v[q] by w_(2^i) for every set bit i of q, so
+// only log2(R) roots are live (the composed form would hold R of them).
+template <int R, int DIR, int OFF, int E>
 __device__ __forceinline__ void pass_twiddle(float2 (&v)[E], const float2* __restrict__ tp, int ns, int k) {
     constexpr int LOGR = ilog2(R);
-    auto root = [&](int i) -> float2 {
-        if constexpr (SROW) return *byte_off(tp + opaque_uniform((int64_t)i * ns), (uint32_t)k * 8u);
-        else return tp[i * ns + k];
-    };
+    auto root = [&](int i) -> float2 { return tp[i * ns + k]; };
     if constexpr (R <= 16) {
         float2 w[R];
         static_for<0, LOGR>([&](auto i) { w[1 << i.value] = root(i.value); });

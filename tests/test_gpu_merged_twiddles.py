@@ -59,3 +59,39 @@ def test_four_step_real(pkg, gpu, l1, l2):
     assert np.linalg.norm(spec.cpu().numpy() - e) <= U * math.sqrt(levels) * np.linalg.norm(e)
     back = pkg.execute_fft_plan(pkg.ExecutionPlan(transform_type="c2r", transform_direction="inverse", **common), spec)
     assert np.linalg.norm(back.cpu().numpy() - x) <= U * math.sqrt(2 * levels) * np.linalg.norm(x)
+
+
+@pytest.mark.parametrize("direction", ["forward", "inverse"])
+@pytest.mark.parametrize("logn", [11, 12, 13, 14, 15])
+def test_lds_32_elements(pkg, gpu, logn, direction):
+    """Remainder radices 2, 4, 8, 16 and 32 after the radix-32 passes, and the
+    last block's rows past a ragged batch."""
+    err = _run(pkg, gpu, 1 << logn, 3, direction, "fft_lds_fused_batch", {"elems": 32}, logn)
+    assert err <= U * math.sqrt(logn), err
+
+
+@pytest.mark.parametrize("logn", [4, 5, 6, 7, 8, 10, 11])
+@pytest.mark.parametrize("batch", [1, 3, 257])
+def test_lds_last_block_rows(pkg, gpu, logn, batch):
+    """Several transforms a block: the threads of rows past the batch load its
+    last row again and store nothing, in each mode."""
+    import torch
+
+    n = 1 << logn
+    x = np.random.default_rng(n + batch).standard_normal((batch, n)).astype(np.float32)
+    xin = torch.from_numpy(x[0] if batch == 1 else x).to(gpu)
+    for elems in (4, 8, 16, 32):
+        if elems == 32 and logn < 11:
+            continue
+        common = dict(n=n, batch=batch, direction="dit", precision="fp32", selection_source="table", reason="test",
+                      fallback=False, executed="fft_lds_fused_batch", block=None, params={"elems": elems}, norm="ortho")
+        spec = pkg.execute_fft_plan(pkg.ExecutionPlan(transform_type="r2c", **common), xin)
+        back = pkg.execute_fft_plan(pkg.ExecutionPlan(transform_type="c2r", transform_direction="inverse", **common),
+                                    spec)
+        cplx = pkg.execute_fft_plan(pkg.ExecutionPlan(**common), xin.to(torch.complex64))
+        e = np.fft.fft(x.astype(np.float64), norm="ortho")
+        tol = U * math.sqrt(2 * (logn + 2))
+        assert np.linalg.norm(cplx.cpu().numpy().reshape(batch, -1) - e) <= tol * np.linalg.norm(e)
+        half = e[:, : n // 2 + 1]
+        assert np.linalg.norm(spec.cpu().numpy().reshape(batch, -1) - half) <= tol * np.linalg.norm(half)
+        assert np.linalg.norm(back.cpu().numpy().reshape(batch, -1) - x) <= tol * np.linalg.norm(x)
