@@ -166,6 +166,19 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
     // values are not line-aligned and take partial-line writes) loses more,
     // so both real modes keep plain stores.
     constexpr bool WT = MODE == 0 && LOGL <= 13 && (STAGED || T >= 16);
+    // Bin rows of L + 1 values start anywhere in a 128-byte line, so the runs
+    // of 32 lanes that lane pairing loads and stores straddle lines.  BINS_OUT
+    // and BINS_IN move the block's bins through LDS instead, every memory
+    // instruction on whole lines, for one more LDS round.
+    // R2C out, with write-through stores of those lines: N = 2^10, B = 65536
+    // (8 elements): 104 -> 99 us, 2^13, B = 8192 (16): 101 -> 97, 2^14, B = 256:
+    // 12.6 -> 11.8; at cores of 2^14 and 2^15 points the one or two blocks of a
+    // CU wait longer in the round than they gain (2^16, B = 1000: 136 -> 143).
+    // C2R in, with 32 elements: N = 2^14, B = 4096: 109.8 -> 104.7, 2^15, B =
+    // 2048: 118.0 -> 112.8; not at 2^15 points (137 -> 144), and with 16
+    // elements or fewer the gain is within 2% and a small batch pays the round.
+    constexpr bool BINS_OUT = MODE == 1 && C::PAIR && LOGL <= 13;
+    constexpr bool BINS_IN = MODE == 2 && C::PAIR && C::LE == 5 && LOGL >= 12 && LOGL <= 14;
     static_assert(!(C::SPLIT && MODE == 1 && C::LE != 5 && !C::PAIR),
                   "16-element r2c kernels without lane pairing stitch whole complex values out of LDS");
     __shared__ float2 lds_raw[NEED_LDS ? (C::LDS_FLOATS + 1) / 2 : 1];
@@ -233,10 +246,52 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             // j = 0 reads is still the bin: v[E-s] belongs to a later pair,
             // and v[s+1], already turned, was kept in `prev`.
             static_assert(R0 == E && NB0 == 1, "lane pairing needs a full radix first pass");
-            const float2* xb = (const float2*)src_v + lrow * (L + 1);
-            static_for<0, E>([&](auto q) { v[q.value] = load_nt(xb + j + q.value * T); });
             const bool jz = j == 0, jh = j == T / 2;
-            const float2 xny = jz ? load_nt(xb + L) : make_float2(0.0f, 0.0f);
+            float2 xny = make_float2(0.0f, 0.0f);
+            if constexpr (BINS_IN) {
+                // in through LDS: element e of the block's TPB * (L + 1) bins is
+                // loaded by lane (e + sh) mod 64, so every load reads whole lines
+                const int64_t first = (int64_t)blockIdx.x * C::TPB;
+                const int here = C::TPB == 1 || rows - first > C::TPB ? C::TPB : (int)(rows - first);
+                const float2* const xb = (const float2*)src_v + first * (L + 1);
+                const int sh = (int)((reinterpret_cast<uintptr_t>(xb) >> 3) & 15);
+                const float2* const xa = xb - sh;  // the line that holds the block's first bin
+                const int e0 = tid - sh;
+                const int end = here * (L + 1);
+                const int own = tl * (L + 1) + j;
+                float2 tail = make_float2(0.0f, 0.0f);
+                auto in_row = [&](auto r) {
+                    const int e = e0 + r.value * C::WG;
+                    return (r.value > 0 || e >= 0) && ((C::TPB == 1 && r.value < E) || e < end);
+                };
+                static_for<0, E + 1>([&](auto r) {
+                    float2& x = r.value == E ? tail : v[r.value % E];
+                    x = make_float2(0.0f, 0.0f);
+                    if (in_row(r)) x = load_nt(byte_off(xa + r.value * C::WG, (uint32_t)tid * 8u));
+                });
+                static_for<0, C::SPLIT ? 2 : 1>([&](auto comp) {
+                    if constexpr (comp.value > 0) __syncthreads();  // the real parts have been read
+                    static_for<0, E + 1>([&](auto r) {
+                        const float2 x = r.value == E ? tail : v[r.value % E];
+                        if (in_row(r)) {
+                            if constexpr (!C::SPLIT) lds[e0 + r.value * C::WG] = x;
+                            else ldsf[e0 + r.value * C::WG] = comp.value == 0 ? x.x : x.y;
+                        }
+                    });
+                    __syncthreads();
+                    static_for<0, E + 1>([&](auto q) {
+                        float2& x = q.value == E ? xny : v[q.value % E];
+                        const int e = q.value == E ? (jz ? own + L : own) : own + q.value * T;
+                        if constexpr (!C::SPLIT) x = lds[e];
+                        else if constexpr (comp.value == 0) x.x = ldsf[e];
+                        else x.y = ldsf[e];
+                    });
+                });
+            } else {
+                const float2* xb = (const float2*)src_v + lrow * (L + 1);
+                static_for<0, E>([&](auto q) { v[q.value] = load_nt(xb + j + q.value * T); });
+                if (jz) xny = load_nt(xb + L);
+            }
             // exp(-2 pi i (j + T*s) / 2L) = tw_real[j] * exp(-2 pi i s / 2E):
             // one table load and compile-time rotations
             const float2 tj = tw_real[j];
@@ -393,7 +448,7 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
         });
         if constexpr ((p < P - 1 || (MODE == 1 && !C::PAIR)) && !C::SPLIT) {
             // every thread has read this pass's inputs (pass 0 of c2r: the partner bins)
-            if constexpr (p > 0 || (MODE == 2 && !C::PAIR) || STAGED) __syncthreads();
+            if constexpr (p > 0 || (MODE == 2 && !C::PAIR) || STAGED || BINS_IN) __syncthreads();
             static_for<0, NB>([&](auto m) {
                 const int b = j + m.value * T;
                 const int base = ((b >> LNS) << (LNS + LR)) + (b & (NS - 1));
@@ -438,26 +493,79 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
         // r2c under lane pairing: v[q] = Z[j + T*q] and the mirror of
         // Z[j + T*q] is the partner lane's v[E-1-q] (own v[E-1-q] for
         // j = T/2, own v[(E-q) mod E] for j = 0), so every bin is stitched
-        // in registers and stored once; thread j = 0 also writes bin L.
+        // in registers and stored once; thread j = 0 also has bin L.  A
+        // transform spans whole waves, and the threads of rows past the batch
+        // hold its last row: every lane swap runs with all lanes of the wave.
         static_assert(C::logr(P - 1) == C::LE, "lane pairing needs a full radix last pass");
-        float2* xo = (float2*)dst_v + row * (L + 1);
         const bool jz = j == 0, jh = j == T / 2;
-        // A transform spans whole waves, so `active` is wave-uniform and the
-        // lane swaps run with every lane of the wave or none.
-        if (active) {
-            const float2 tj = tw_real[j];  // tw_real[j + T*s] = tj * exp(-2 pi i s / 2E)
-            static_for<0, E / 2>([&](auto ss) {
-                constexpr int s = ss.value;
-                constexpr int sb = E - 1 - s;
-                const float2 a = v[s], b = v[sb];
-                const float2 pa = swap_halves(b), pb = swap_halves(a);
-                const float2 ma = jz ? v[(E - s) % E] : (jh ? b : pa);
-                const float2 mb = jz ? v[s + 1] : (jh ? a : pb);
-                xo[j + s * T] = r2c_bin(a, ma, rot<2 * E, s, -1>(tj), scale, s == 0 && jz);
-                xo[j + sb * T] = r2c_bin(b, mb, rot<2 * E, sb, -1>(tj), scale, false);
-                __builtin_amdgcn_sched_barrier(0);
+        const float2 tj = tw_real[j];  // tw_real[j + T*s] = tj * exp(-2 pi i s / 2E)
+        const float2 ny = r2c_bin(v[0], v[0], tw_real[L], scale, true);  // bin L, kept by j = 0
+        float2 prev = v[0];  // Z of element (E - s) mod E, which an earlier pair may have turned into a bin
+        float2* const xo = (float2*)dst_v + row * (L + 1) + j;
+        static_for<0, E / 2>([&](auto ss) {
+            constexpr int s = ss.value;
+            constexpr int sb = E - 1 - s;
+            const float2 a = v[s], b = v[sb];
+            const float2 pa = swap_halves(b), pb = swap_halves(a);
+            const float2 ma = jz ? prev : (jh ? b : pa);
+            const float2 mb = jz ? v[s + 1] : (jh ? a : pb);
+            const float2 xa = r2c_bin(a, ma, rot<2 * E, s, -1>(tj), scale, s == 0 && jz);
+            const float2 xb = r2c_bin(b, mb, rot<2 * E, sb, -1>(tj), scale, false);
+            prev = b;
+            if constexpr (BINS_OUT) {
+                v[s] = xa;
+                v[sb] = xb;
+                // computed here: sunk below the exchange's first barrier, the
+                // imaginary parts would keep every pair's operands in registers
+                asm volatile("" : "+v"(v[s].x), "+v"(v[s].y), "+v"(v[sb].x), "+v"(v[sb].y));
+            } else if (active) {
+                xo[s * T] = xa;
+                xo[sb * T] = xb;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (BINS_OUT) {
+            // out through LDS: element e of the block's TPB * (L + 1) bins goes to
+            // lane (e + sh) mod 64, so every store instruction writes whole lines
+            const int64_t first = (int64_t)blockIdx.x * C::TPB;
+            const int here = C::TPB == 1 || rows - first > C::TPB ? C::TPB : (int)(rows - first);
+            float2* const xb = (float2*)dst_v + first * (L + 1);
+            const int sh = (int)((reinterpret_cast<uintptr_t>(xb) >> 3) & 15);
+            float2* const xa = xb - sh;  // the line that holds the block's first bin
+            const int e0 = tid - sh;
+            const int own = tl * (L + 1) + j;
+            float2 tail;
+            static_for<0, C::SPLIT ? 2 : 1>([&](auto comp) {
+                __syncthreads();  // the previous readers of this LDS are done
+                static_for<0, E>([&](auto q) {
+                    if constexpr (!C::SPLIT) lds[own + q.value * T] = v[q.value];
+                    else ldsf[own + q.value * T] = comp.value == 0 ? v[q.value].x : v[q.value].y;
+                });
+                // bin L from j = 0; the other threads write their element 0 again
+                const int ei = jz ? own + L : own;
+                const float2 xe = make_float2(jz ? ny.x : v[0].x, jz ? ny.y : v[0].y);
+                if constexpr (!C::SPLIT) lds[ei] = xe;
+                else ldsf[ei] = comp.value == 0 ? xe.x : xe.y;
+                __syncthreads();
+                static_for<0, E + 1>([&](auto r) {
+                    // within the array: e0 >= -15, and the last round is past its end in most lanes
+                    const int e = r.value == 0 ? (e0 < 0 ? 0 : e0)
+                                               : (r.value == E ? (e0 < C::TPB ? e0 + E * C::WG : 0) : e0 + r.value * C::WG);
+                    float2& x = r.value == E ? tail : v[r.value % E];
+                    if constexpr (!C::SPLIT) x = lds[e];
+                    else if constexpr (comp.value == 0) x.x = ldsf[e];
+                    else x.y = ldsf[e];
+                });
             });
-            if (jz) xo[L] = r2c_bin(v[0], v[0], tw_real[L], scale, true);
+            const int end = here * (L + 1);
+            static_for<0, E + 1>([&](auto r) {
+                const int e = e0 + r.value * C::WG;
+                if ((r.value > 0 || e >= 0) && ((C::TPB == 1 && r.value < E) || e < end))
+                    store_out<true>(byte_off(xa + r.value * C::WG, (uint32_t)tid * 8u),
+                                    r.value == E ? tail : v[r.value % E]);
+            });
+        } else if (active && jz) {
+            xo[L] = ny;
         }
     } else if constexpr (MODE == 1 && C::SPLIT) {
         // r2c with 32 elements per thread and no lane pairing (the last

@@ -1,0 +1,70 @@
+"""Bin rows moved in whole 128-byte lines (the real modes of the LDS kernel):
+rows of n/2 + 1 bins that start anywhere in a line, several rows a block, a
+ragged last block and nothing written outside the rows, against 64-bit numpy.
+
+The bound is that of the transform's own rounding: below u per radix-2 level
+and for the stitch (u = 2^-24), so u sqrt(log2 n + 2) in the 2-norm; a bin in
+a neighbour's place gives an error of order one.
+"""
+import math
+
+import numpy as np
+import pytest
+
+from kunlunxin_fft_amd import native
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+GUARD = 32  # bins or samples around the rows that must stay as they are
+
+# (log2 n, elements per thread): 8 and 16 elements with one and with several
+# transforms a block, float2 and split exchange, and 32 elements; for C2R the
+# first and last core length whose bins come in through LDS and their neighbours
+CASES = [(10, 8), (11, 8), (12, 8), (11, 16), (12, 16), (13, 16), (14, 16), (15, 16),
+         (12, 32), (13, 32), (14, 32), (15, 32), (16, 32)]
+
+
+def _plan(n, batch, kind, elems):
+    return native.NativePlan(n, batch, kind, "forward" if kind == "r2c" else "inverse", norm="ortho",
+                             flow=native.FLOW_LDS_FUSED, params=[elems])
+
+
+@pytest.mark.parametrize("batch,shift", [(1, 0), (3, 1), (5, 8), (2, 15)])
+@pytest.mark.parametrize("logn,elems", CASES)
+def test_bin_rows(gpu, logn, elems, batch, shift):
+    import torch
+
+    n, m = 1 << logn, (1 << (logn - 1)) + 1
+    x = np.random.default_rng(100 * logn + elems + shift).standard_normal((batch, n)).astype(np.float32)
+    e = np.fft.rfft(x.astype(np.float64), norm="ortho")
+    tol = U * math.sqrt(logn + 2)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    plan = _plan(n, batch, "r2c", elems)
+    xin = torch.from_numpy(x).to(gpu)
+    buf = torch.full((GUARD + shift + batch * m + GUARD,), 7.0 + 5.0j, dtype=torch.complex64, device=gpu)
+    first = GUARD + shift
+    plan.execute(xin.data_ptr(), buf[first:].data_ptr(), stream)
+    torch.cuda.synchronize()
+    got = buf.cpu().numpy()
+    assert np.all(got[:first] == 7 + 5j) and np.all(got[first + batch * m:] == 7 + 5j)
+    got = got[first:first + batch * m].reshape(batch, m)
+    for r in range(batch):
+        assert np.linalg.norm(got[r] - e[r]) <= tol * np.linalg.norm(e[r]), r
+
+    plan = _plan(n, batch, "c2r", elems)
+    spec = np.full((GUARD + shift + batch * m + GUARD,), np.nan + 1j * np.nan, dtype=np.complex64)
+    bins = e.astype(np.complex64)
+    bins[:, 0] += 3j  # the imaginary parts of bins 0 and n/2 are ignored
+    bins[:, -1] -= 2j
+    spec[first:first + batch * m] = bins.reshape(-1)
+    sin = torch.from_numpy(spec).to(gpu)
+    out = torch.full((batch * n + GUARD,), 7.0, dtype=torch.float32, device=gpu)
+    plan.execute(sin[first:].data_ptr(), out.data_ptr(), stream)
+    torch.cuda.synchronize()
+    back = out.cpu().numpy()
+    assert np.all(back[batch * n:] == 7.0)
+    back = back[:batch * n].reshape(batch, n)
+    for r in range(batch):
+        assert np.linalg.norm(back[r] - x[r]) <= (tol + U) * np.linalg.norm(x[r]), r  # + the bins' own rounding
