@@ -27,8 +27,9 @@
 // twiddles ran N = 2^20, B = 64 in 345 us against 380.  Multiplying pass 1's
 // outputs by the twiddle and pass 2's inputs by pass twiddles took 3151 vector
 // instructions per thread over the two passes at 1024 points and 32 elements;
-// merged they take 2522.  N = 2^20, B = 64: 376 -> 362 us; 2^16, B = 256: 87 ->
-// 83; C2R 2^18, B = 256: 195 -> 181; R2C: 226 -> 217; 2^16, B = 32: 15.8 -> 14.3.
+// merged they take 2745.  N = 2^20, B = 64: 375 -> 364 us; 2^16, B = 256: 85.1
+// -> 81.2; C2R 2^18, B = 256: 192 -> 179; R2C: 240 -> 236; 2^16, B = 32: 14.7 ->
+// 14.0.
 // Those roots are products of a Stockham root, from a per-pass table (rows
 // W^k, W^2k, W^4k, ...) that both passes have, and of W_N^(2^t k1), t < log2
 // N2, from one row per t of N1 entries: both loads are contiguous or shared
@@ -179,12 +180,6 @@ struct PassRoots {
         });
     }
 };
-// Levels of a twiddled radix-2^lr DFT that take the short butterfly: as many
-// as keep the error against 64 bits at or below that of a separate product by
-// W_N^(n2*k1).  Pass 2's roots are rounded products, so it takes one less.
-constexpr int col_six(int lr, int kind) {
-    return lr >= 5 ? 3 - kind : (lr == 4 ? 2 - kind : (lr == 3 ? 1 : 0));
-}
 
 // Pass-0 operands of one column group: s = the group's first element of the
 // transform (wave-uniform), lane (c, j) reads rows j + m*T + q*L/R0 of column c.
@@ -250,11 +245,11 @@ __device__ __forceinline__ void col_passes(float2 (&v)[C::E], float2* lds, int c
         }
         static_for<0, NB>([&](auto m) {
             if constexpr (p == 0) {
-                dft_dit<R, DIR, m.value * R, KIND == 1, col_six(LR, KIND)>(v, r0);
+                dft_dit<R, DIR, m.value * R, KIND == 1>(v, r0);
             } else {
                 float2 r[LR];
                 roots.template load<p, m.value>(r, j + m.value * T);
-                dft_dit<R, DIR, m.value * R, true, col_six(LR, KIND)>(v, r);
+                dft_dit<R, DIR, m.value * R, true>(v, r);
             }
         });
         if constexpr (p < P - 1 && !C::SPLIT) {

@@ -91,13 +91,12 @@ struct LdsCfg {
     // themselves).
     static constexpr bool PAIR =
         LE >= 3 && T >= 64 && (MODE == 2 || (MODE == 1 && sched_logr(LOGL, LE, P - 1, RF) == LE));
-    // Pass twiddles merged into the butterflies (dft_dit, one level short) with
-    // 32 elements per thread: 10-15% fewer vector instructions (2^13: 1939 ->
-    // 1642, 2^15: 2324 -> 2100), N = 2^13 of 256 MiB 90 -> 87 us, 2^14 97 -> 95,
-    // 2^14, B = 256 20 -> 19.2, R2C 2^16 125 -> 122.  Up to 16 elements the
-    // products cost little more (272 operations a pass against 256) and both
-    // forms run alike (N = 4096: 82 us); at 1024 points the merged form spills
-    // (81 -> 95 us).
+    // Pass twiddles merged into the butterflies (dft_dit) with 32 elements per
+    // thread: 7-12% fewer vector instructions (2^13: 1939 -> 1705, 2^15: 2324 ->
+    // 2163), N = 2^13 of 512 MiB 180 -> 176 us, 2^14, B = 256 19.2 -> 18.7, R2C
+    // 2^16, B = 1024 135 -> 132.  Up to 16 elements both forms take the same
+    // number of operations and run alike (N = 4096: 82 us); at 1024 points the
+    // merged form spills (81 -> 95 us).
     static constexpr bool MERGED = LE == 5 && LOGL >= 11;
     static constexpr int logr(int p) { return sched_logr(LOGL, LE, p, RF); }
     static constexpr int lns(int p) { return sched_lns_rf(LOGL, LE, p, RF); }
@@ -440,7 +439,7 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             if constexpr (C::MERGED) {
                 float2 r[LR > 0 ? LR : 1];
                 if constexpr (NS > 1) pass_roots<LR, C::WG == 1024>(r, tw + TW_OFF, NS, k);
-                dft_dit<R, DIR, m.value * R, (NS > 1), (LR >= 3 ? 1 : 0)>(v, r);
+                dft_dit<R, DIR, m.value * R, (NS > 1)>(v, r);
             } else {
                 if constexpr (NS > 1) pass_twiddle<R, DIR, m.value * R>(v, tw + TW_OFF, NS, k);
                 dft<R, DIR, m.value * R, 1>(v);

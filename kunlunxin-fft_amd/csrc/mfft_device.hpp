@@ -148,29 +148,32 @@ __device__ __forceinline__ void dft(float2 (&v)[E]) {
 // and its products with the compile-time roots m < 2^(l-2); the other half
 // differs by a factor -+i, which a swap of operands applies.
 //
-// A butterfly is four FMAs for a + w b and four more for a - w b, or two:
-// 2 a - (a + w b), which also carries the first result's rounding.  This
-// short form is taken in the first SIX levels of a twiddled DFT.  Products of
-// the inputs by w^q and then a decimation-in-frequency network take 272
-// operations at R = 16 and 776 at R = 32 (only the log2 R loaded roots fit the
-// registers beside 32 values); merged it is 256 and 652 with one level short,
-// with an error against 64 bits 0-5% smaller.  With every level short (208
-// and 524) the error would be 3-6% larger, and with the product t = w b and
-// a +- t for the long form 0-2%.
-template <int DIR, bool ROT, bool SIX_OPS>
+// A butterfly is four FMAs for a + w b and four for a - w b.  Deriving the
+// second as 2 a - (a + w b) would take two, but where a + w b overflows or a is
+// infinite it loses a - w b as well, and with it half of the bins that depend on
+// the two.  For the same reason the last level takes the product t = w b first:
+// a + Re(w) b alone can leave the range where a + w b is inside it.
+// Products of the inputs by w^q and then a decimation-in-frequency network take
+// 272 operations at R = 16 and 776 at R = 32 (only the log2 R loaded roots fit
+// the registers beside 32 values); merged it is 272 and 684, with an error
+// against 64 bits 0.6-2% smaller (with the product first on every level it
+// would be 1% larger).
+template <int DIR, bool ROT, bool LAST>
 __device__ __forceinline__ void butterfly(float2& a, float2& b, float wx, float wy) {
     const float q = DIR < 0 ? wy : -wy;
     // w b = (xx b.x + xy b.y, yx b.x + yy b.y), times DIR i with ROT
     const float xx = !ROT ? wx : (DIR < 0 ? q : -q), xy = !ROT ? -q : (DIR < 0 ? wx : -wx);
     const float yx = !ROT ? q : (DIR < 0 ? -wx : wx), yy = !ROT ? wx : (DIR < 0 ? q : -q);
-    const float sx = fmaf(xy, b.y, fmaf(xx, b.x, a.x));
-    const float sy = fmaf(yy, b.y, fmaf(yx, b.x, a.y));
-    if constexpr (SIX_OPS) {
-        b = make_float2(fmaf(2.0f, a.x, -sx), fmaf(2.0f, a.y, -sy));
+    if constexpr (LAST) {
+        const float2 t = make_float2(fmaf(xy, b.y, xx * b.x), fmaf(yy, b.y, yx * b.x));
+        b = csub(a, t);
+        a = cadd(a, t);
     } else {
+        const float sx = fmaf(xy, b.y, fmaf(xx, b.x, a.x));
+        const float sy = fmaf(yy, b.y, fmaf(yx, b.x, a.y));
         b = make_float2(fmaf(-xy, b.y, fmaf(-xx, b.x, a.x)), fmaf(-yy, b.y, fmaf(-yx, b.x, a.y)));
+        a = make_float2(sx, sy);
     }
-    a = make_float2(sx, sy);
 }
 // the same for w = 1 (times DIR i with ROT)
 template <int DIR, bool ROT>
@@ -183,7 +186,7 @@ __device__ __forceinline__ void butterfly1(float2& a, float2& b) {
 // v[OFF + q], q in [0, R): natural order in and out.  r[i] = w^(2^i) as
 // forward-table roots (DIR = +1 takes their conjugates); TW = false: w = 1,
 // r is not read.
-template <int R, int DIR, int OFF, bool TW, int SIX, int E, int NR>
+template <int R, int DIR, int OFF, bool TW, int E, int NR>
 __device__ __forceinline__ void dft_dit(float2 (&v)[E], const float2 (&r)[NR]) {
     static_assert(R >= 1 && (R & (R - 1)) == 0, "radix must be a power of two");
     constexpr int LOGR = ilog2(R);
@@ -203,8 +206,7 @@ __device__ __forceinline__ void dft_dit(float2 (&v)[E], const float2 (&r)[NR]) {
                         if constexpr (!TW && m == 0)
                             butterfly1<DIR, rotated.value>(v[i0 + q.value], v[i0 + q.value + h]);
                         else
-                            butterfly<DIR, rotated.value, TW && (l <= SIX)>(v[i0 + q.value], v[i0 + q.value + h], w.x,
-                                                                            w.y);
+                            butterfly<DIR, rotated.value, l == LOGR>(v[i0 + q.value], v[i0 + q.value + h], w.x, w.y);
                     });
                 };
                 const float2 w = rot<(1 << l), m, -1>(TW ? r[TW ? LOGR - l : 0] : make_float2(1.0f, 0.0f));

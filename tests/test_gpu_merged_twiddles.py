@@ -95,3 +95,60 @@ def test_lds_last_block_rows(pkg, gpu, logn, batch):
         half = e[:, : n // 2 + 1]
         assert np.linalg.norm(spec.cpu().numpy().reshape(batch, -1) - half) <= tol * np.linalg.norm(half)
         assert np.linalg.norm(back.cpu().numpy().reshape(batch, -1) - x) <= tol * np.linalg.norm(x)
+
+
+MAX = float(np.finfo(np.float32).max)
+RANGE_PLANS = [("fft_lds_fused_batch", 12, {"elems": 32}), ("fft_lds_fused_batch", 13, {"elems": 32}),
+               ("fft_lds_fused_batch", 14, {"elems": 32}), ("fft_lds_fused_batch", 15, {"elems": 32}),
+               ("fft_lds_fused_batch", 12, {"elems": 16}), ("fft_four_step_batch", 14, {"n1": 64}),
+               ("fft_four_step_batch", 16, {"n1": 256}), ("fft_four_step_batch", 18, {"n1": 512}),
+               ("fft_four_step_batch", 20, {"n1": 1024}), ("fft_four_step_batch", 20, {"n1": 1024, "schedule": 3})]
+
+
+def _unscaled(pkg, gpu, executed, logn, params, x):
+    import torch
+
+    plan = pkg.ExecutionPlan(n=1 << logn, batch=len(x), direction="dit", precision="fp32", selection_source="table",
+                             reason="test", fallback=False, executed=executed, block=None, params=params, norm="none")
+    x = torch.from_numpy(x.astype(np.complex64)).to(gpu)
+    return pkg.execute_fft_plan(plan, x[0] if len(x) == 1 else x).cpu().numpy().reshape(x.shape)
+
+
+@pytest.mark.parametrize("executed,logn,params", RANGE_PLANS)
+def test_overflow_stays_in_its_bins(pkg, gpu, executed, logn, params):
+    """A tone whose own bin exceeds the float range 2^d to 2^(d+1) times: the
+    first partial sums that overflow are those of n / 2^d samples, which only
+    the 2^d bins k0 + i n / 2^d are computed from; the rest stays finite."""
+    n, k0 = 1 << logn, 5
+    for d in range(5):
+        x = (1.5 * 2.0 ** d * MAX / n) * np.exp(2j * np.pi * k0 * np.arange(n) / n)
+        y = _unscaled(pkg, gpu, executed, logn, params, x[None])[0]
+        lost = np.flatnonzero(~(np.isfinite(y.real) & np.isfinite(y.imag)))
+        assert set(lost) <= set((k0 + np.arange(1 << d) * (n >> d)) % n) and k0 in lost, (d, lost[:8])
+
+
+@pytest.mark.parametrize("executed,logn,params", RANGE_PLANS)
+def test_infinite_first_sample(pkg, gpu, executed, logn, params):
+    """x[0] enters every bin with factor 1: an infinite real part makes every
+    real part infinite and leaves the imaginary parts finite."""
+    x = np.full((1, 1 << logn), 0.5 + 0j)
+    x[0, 0] = np.inf
+    y = _unscaled(pkg, gpu, executed, logn, params, x)
+    assert np.all(np.isposinf(y.real)) and np.all(np.isfinite(y.imag))
+
+
+@pytest.mark.parametrize("executed,logn,params", RANGE_PLANS)
+def test_largest_values_in_range(pkg, gpu, executed, logn, params):
+    """Bins up to 0.999 of the largest float come out, whatever the partial
+    sums on the way to them."""
+    n, batch = 1 << logn, max(1, (1 << 20) >> logn)
+    rng = np.random.default_rng(logn)
+    x = rng.standard_normal((batch, n)) + 1j * rng.standard_normal((batch, n))
+    e = np.fft.fft(x)
+    top = 0.999 * MAX / np.maximum(np.abs(e.real).max(-1), np.abs(e.imag).max(-1))[:, None]
+    y = _unscaled(pkg, gpu, executed, logn, params, x * top)
+    assert np.all(np.isfinite(y.real)) and np.all(np.isfinite(y.imag))
+    e = e * top / MAX
+    y = y.astype(np.complex128) / MAX
+    # one rounding for the samples beside those of the network
+    assert np.linalg.norm(y - e) <= U * math.sqrt(logn + 1) * np.linalg.norm(e)
