@@ -186,14 +186,6 @@ bool is_stage_flow(int f) {
            f == MFFT_FLOW_RADIX4_DIF;
 }
 
-// LDS_FUSED elements per thread where the caller leaves the choice.  Real
-// transforms on a core of 2^13 or 2^14 points take 32 once the launch fills the
-// card: fewer passes (3 against 4) and half the threads.  ELEMS_FIGURES
-int default_elems(int logc, bool real, int64_t batch) {
-    if (real && (logc == 13 || logc == 14) && (batch << logc) >= ((int64_t)1 << 23)) return 32;
-    return mfft::lds_default_elems(logc);
-}
-
 // Alignment of a caller workspace and of the ws_b offset inside it.
 constexpr int64_t kWorkAlign = 256;
 
@@ -429,7 +421,7 @@ int mfft_plan_create_ex(mfft_plan** out, int64_t n, int64_t batch, int transform
                             "elements per thread (32 from 2^10; 2^13, 2^14: 16 or 32; 2^15: 32) "
                             "(got core length %lld, elements %d)",
                             mfft::kMaxLdsLog2, (long long)core_n, prm[0]);
-            elems = prm[0] ? prm[0] : default_elems(logc, real, batch);
+            elems = prm[0] ? prm[0] : mfft::lds_default_elems(logc);
             block = mfft::lds_threads_per_block(logc, elems);
             if (prm[1] > mfft::kMaxStagger)
                 return fail(MFFT_ERR_VALUE, "LDS_FUSED start stagger params[1]=%d exceeds %d", prm[1],

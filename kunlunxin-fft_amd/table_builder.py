@@ -324,14 +324,6 @@ def real_candidates(n: int, b: int, transform_type: str, space):
             if 1 in space.lds_staged and e != 32 and core // min(e, core) < 16:
                 out.append((f"lds_e{e}_st", "fft_lds_fused" + sfx, 256, {"elems": e, "stage": 1},
                             ("lds-resident", "stockham-radix16", "lds-stockham-single-pass")))
-        # no element count: the library's choice for the core and the batch, 32
-        # elements at these cores once the launch fills the card (the runner
-        # maps an explicit 32 to 16 below a 32768-point core)
-        if logc in (13, 14) and n * b >= (1 << 24):
-            for stg in space.lds_stagger if 0 in space.lds_stagger else (0, *space.lds_stagger):
-                out.append(("lds_auto" + (f"_s{stg}" if stg else ""), "fft_lds_fused" + sfx, 256,
-                            {"stagger": stg} if stg else {},
-                            ("lds-resident", "stockham-radix16", "lds-stockham-single-pass")))
     if 256 <= core and core * 2 >= space.fourstep_min_n:
         for n1 in space.fourstep_n1:
             n2 = core // n1

@@ -68,3 +68,27 @@ def test_bin_rows(gpu, logn, elems, batch, shift):
     back = back[:batch * n].reshape(batch, n)
     for r in range(batch):
         assert np.linalg.norm(back[r] - x[r]) <= (tol + U) * np.linalg.norm(x[r]), r  # + the bins' own rounding
+
+
+@pytest.mark.parametrize("kind", ["r2c", "c2r"])
+@pytest.mark.parametrize("logn", [14, 15])
+def test_default_kernel_is_the_same_at_every_batch(gpu, logn, kind):
+    """Without an element count a row comes from the same kernel, so with the
+    same bits, whatever the batch around it."""
+    import torch
+
+    n, batch = 1 << logn, 1 << (24 - logn)
+    shape = (batch, n) if kind == "r2c" else (batch, n + 2)  # a row of samples, or of n/2 + 1 bins
+    x = torch.from_numpy(np.random.default_rng(logn).standard_normal(shape).astype(np.float32)).to(gpu)
+    stream = torch.cuda.current_stream().cuda_stream
+    rows, elems = [], []
+    for b in (1, batch):
+        plan = native.NativePlan(n, b, kind, "forward" if kind == "r2c" else "inverse", norm="ortho",
+                                 flow=native.FLOW_LDS_FUSED)
+        out = torch.empty((b, n + 2 if kind == "r2c" else n), dtype=torch.float32, device=gpu)
+        plan.execute(x.data_ptr(), out.data_ptr(), stream)
+        torch.cuda.synchronize()
+        rows.append(out[0].clone())
+        elems.append(plan.info.elems_per_thread)
+    assert elems[0] == elems[1], elems
+    assert torch.equal(rows[0], rows[1])
