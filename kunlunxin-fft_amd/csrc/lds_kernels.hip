@@ -166,18 +166,15 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
     // so both real modes keep plain stores.
     constexpr bool WT = MODE == 0 && LOGL <= 13 && (STAGED || T >= 16);
     // Bin rows of L + 1 values start anywhere in a 128-byte line, so the runs
-    // of 32 lanes that lane pairing loads and stores straddle lines.  BINS_OUT
-    // and BINS_IN move the block's bins through LDS instead, every memory
-    // instruction on whole lines, for one more LDS round.
-    // R2C out, with write-through stores of those lines: N = 2^10, B = 65536
-    // (8 elements): 104 -> 99 us, 2^13, B = 8192 (16): 101 -> 97, 2^14, B = 256:
-    // 12.6 -> 11.8; at cores of 2^14 and 2^15 points the one or two blocks of a
-    // CU wait longer in the round than they gain (2^16, B = 1000: 136 -> 143).
-    // C2R in, with 32 elements: N = 2^14, B = 4096: 109.8 -> 104.7, 2^15, B =
-    // 2048: 118.0 -> 112.8; not at 2^15 points (137 -> 144), and with 16
-    // elements or fewer the gain is within 2% and a small batch pays the round.
+    // of 32 lanes that lane pairing stores straddle lines.  BINS_OUT moves the
+    // block's bins through LDS instead, every memory instruction on whole lines,
+    // for one more LDS round, with write-through stores of those lines: N = 2^10,
+    // B = 65536 (8 elements): 104 -> 99 us, 2^13, B = 8192 (16): 101 -> 97; at
+    // cores of 2^14 and 2^15 points the one or two blocks of a CU wait longer in
+    // the round than they gain (2^16, B = 1000: 136 -> 143).  The same for the
+    // C2R bins on the way in, with 32 elements, took 10% more at N = 2^13 up to B
+    // = 512 and 3% more past the caches, and 2-4% more at 2^14.
     constexpr bool BINS_OUT = MODE == 1 && C::PAIR && LOGL <= 13;
-    constexpr bool BINS_IN = MODE == 2 && C::PAIR && C::LE == 5 && LOGL >= 12 && LOGL <= 14;
     static_assert(!(C::SPLIT && MODE == 1 && C::LE != 5 && !C::PAIR),
                   "16-element r2c kernels without lane pairing stitch whole complex values out of LDS");
     __shared__ float2 lds_raw[NEED_LDS ? (C::LDS_FLOATS + 1) / 2 : 1];
@@ -247,50 +244,9 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             static_assert(R0 == E && NB0 == 1, "lane pairing needs a full radix first pass");
             const bool jz = j == 0, jh = j == T / 2;
             float2 xny = make_float2(0.0f, 0.0f);
-            if constexpr (BINS_IN) {
-                // in through LDS: element e of the block's TPB * (L + 1) bins is
-                // loaded by lane (e + sh) mod 64, so every load reads whole lines
-                const int64_t first = (int64_t)blockIdx.x * C::TPB;
-                const int here = C::TPB == 1 || rows - first > C::TPB ? C::TPB : (int)(rows - first);
-                const float2* const xb = (const float2*)src_v + first * (L + 1);
-                const int sh = (int)((reinterpret_cast<uintptr_t>(xb) >> 3) & 15);
-                const float2* const xa = xb - sh;  // the line that holds the block's first bin
-                const int e0 = tid - sh;
-                const int end = here * (L + 1);
-                const int own = tl * (L + 1) + j;
-                float2 tail = make_float2(0.0f, 0.0f);
-                auto in_row = [&](auto r) {
-                    const int e = e0 + r.value * C::WG;
-                    return (r.value > 0 || e >= 0) && ((C::TPB == 1 && r.value < E) || e < end);
-                };
-                static_for<0, E + 1>([&](auto r) {
-                    float2& x = r.value == E ? tail : v[r.value % E];
-                    x = make_float2(0.0f, 0.0f);
-                    if (in_row(r)) x = load_nt(byte_off(xa + r.value * C::WG, (uint32_t)tid * 8u));
-                });
-                static_for<0, C::SPLIT ? 2 : 1>([&](auto comp) {
-                    if constexpr (comp.value > 0) __syncthreads();  // the real parts have been read
-                    static_for<0, E + 1>([&](auto r) {
-                        const float2 x = r.value == E ? tail : v[r.value % E];
-                        if (in_row(r)) {
-                            if constexpr (!C::SPLIT) lds[e0 + r.value * C::WG] = x;
-                            else ldsf[e0 + r.value * C::WG] = comp.value == 0 ? x.x : x.y;
-                        }
-                    });
-                    __syncthreads();
-                    static_for<0, E + 1>([&](auto q) {
-                        float2& x = q.value == E ? xny : v[q.value % E];
-                        const int e = q.value == E ? (jz ? own + L : own) : own + q.value * T;
-                        if constexpr (!C::SPLIT) x = lds[e];
-                        else if constexpr (comp.value == 0) x.x = ldsf[e];
-                        else x.y = ldsf[e];
-                    });
-                });
-            } else {
-                const float2* xb = (const float2*)src_v + lrow * (L + 1);
-                static_for<0, E>([&](auto q) { v[q.value] = load_nt(xb + j + q.value * T); });
-                if (jz) xny = load_nt(xb + L);
-            }
+            const float2* xb = (const float2*)src_v + lrow * (L + 1);
+            static_for<0, E>([&](auto q) { v[q.value] = load_nt(xb + j + q.value * T); });
+            if (jz) xny = load_nt(xb + L);
             // exp(-2 pi i (j + T*s) / 2L) = tw_real[j] * exp(-2 pi i s / 2E):
             // one table load and compile-time rotations
             const float2 tj = tw_real[j];
@@ -447,7 +403,7 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
         });
         if constexpr ((p < P - 1 || (MODE == 1 && !C::PAIR)) && !C::SPLIT) {
             // every thread has read this pass's inputs (pass 0 of c2r: the partner bins)
-            if constexpr (p > 0 || (MODE == 2 && !C::PAIR) || STAGED || BINS_IN) __syncthreads();
+            if constexpr (p > 0 || (MODE == 2 && !C::PAIR) || STAGED) __syncthreads();
             static_for<0, NB>([&](auto m) {
                 const int b = j + m.value * T;
                 const int base = ((b >> LNS) << (LNS + LR)) + (b & (NS - 1));

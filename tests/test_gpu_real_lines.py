@@ -1,6 +1,6 @@
-"""Bin rows moved in whole 128-byte lines (the real modes of the LDS kernel):
-rows of n/2 + 1 bins that start anywhere in a line, several rows a block, a
-ragged last block and nothing written outside the rows, against 64-bit numpy.
+"""Bin rows of n/2 + 1 values, which start anywhere in a 128-byte line, in the
+real modes of the LDS kernel: several rows a block, a ragged last block and
+nothing written outside the rows, against 64-bit numpy.
 
 The bound is that of the transform's own rounding: below u per radix-2 level
 and for the stitch (u = 2^-24), so u sqrt(log2 n + 2) in the 2-norm; a bin in
@@ -19,8 +19,7 @@ U = 2.0 ** -24
 GUARD = 32  # bins or samples around the rows that must stay as they are
 
 # (log2 n, elements per thread): 8 and 16 elements with one and with several
-# transforms a block, float2 and split exchange, and 32 elements; for C2R the
-# first and last core length whose bins come in through LDS and their neighbours
+# transforms a block, float2 and split exchange, and 32 elements
 CASES = [(10, 8), (11, 8), (12, 8), (11, 16), (12, 16), (13, 16), (14, 16), (15, 16),
          (12, 32), (13, 32), (14, 32), (15, 32), (16, 32)]
 
