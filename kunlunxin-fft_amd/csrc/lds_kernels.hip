@@ -32,7 +32,8 @@
 //      (16 or 32 elements per thread and whole waves per transform: in
 //      registers across lane pairs, the remainder radix running first; 32
 //      elements and 32 lanes per transform: through the output row) and
-//      writes the n/2+1 bins with the scale
+//      writes the n/2+1 bins with the scale (lane-paired, core up to 2^12, a
+//      launch past the L2s: through LDS, in whole 128-byte lines)
 //   2  c2r: the pre-twiddle of kernels.py:1180-1229 is applied while loading
 //      the n/2+1 bins; the inverse core writes the n real samples as n/2
 //      complex pairs with scale 2*norm_scale
@@ -95,9 +96,9 @@ struct LdsCfg {
     // thread: 7-12% fewer vector instructions (2^13: 1939 -> 1705, 2^15: 2324 ->
     // 2163), N = 2^13 of 512 MiB 180 -> 176 us, 2^14, B = 256 19.2 -> 18.7, R2C
     // 2^16, B = 1024 135 -> 132.  Up to 16 elements both forms take the same
-    // number of operations and run alike (N = 4096: 82 us); at 1024 points the
-    // merged form spills (81 -> 95 us).
-    static constexpr bool MERGED = LE == 5 && LOGL >= 11;
+    // number of operations and run alike (N = 4096: 82 us); at 1024 points, and
+    // in r2c at 2^11 and 2^12, the merged form spills (1024: 81 -> 95 us).
+    static constexpr bool MERGED = LE == 5 && LOGL >= (MODE == 1 ? 13 : 11);
     static constexpr int logr(int p) { return sched_logr(LOGL, LE, p, RF); }
     static constexpr int lns(int p) { return sched_lns_rf(LOGL, LE, p, RF); }
 };
@@ -139,7 +140,11 @@ __device__ __forceinline__ float2 swap_halves(float2 x) {
 // core; L + 1 bins per row of the R2C output and the C2R input); they come
 // in and go out through LDS, lane-consecutive, instead of straight between
 // HBM and the registers of pass 0 / the last pass or the stitch.
-template <int LOGL, int LOGE, int DIR, int MODE, bool STAGED = false>
+// LINES (lane-paired r2c, launch_r2c): bin rows of L + 1 values start anywhere
+// in a 128-byte line, so the runs of 32 lanes that lane pairing stores straddle
+// lines; the block's bins go out through LDS instead, written through in whole
+// lines, for one more LDS round.
+template <int LOGL, int LOGE, int DIR, int MODE, bool STAGED = false, bool LINES = false>
 __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE, MODE>::MIN_WAVES)) void lds_fft_kernel(
     const void* __restrict__ src_v, void* __restrict__ dst_v, const float2* __restrict__ tw,
     const float2* __restrict__ tw_real, int64_t rows, float scale, int stag_wave, int stag_cus, int stag_n) {
@@ -163,18 +168,10 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
     // kernel itself is 2-3% slower with them; C2R's real rows gain by
     // themselves but the transform after them (R2C, whose bin rows of L + 1
     // values are not line-aligned and take partial-line writes) loses more,
-    // so both real modes keep plain stores.
+    // so both real modes keep plain stores, except R2C's whole lines (LINES).
     constexpr bool WT = MODE == 0 && LOGL <= 13 && (STAGED || T >= 16);
-    // Bin rows of L + 1 values start anywhere in a 128-byte line, so the runs
-    // of 32 lanes that lane pairing stores straddle lines.  BINS_OUT moves the
-    // block's bins through LDS instead, every memory instruction on whole lines,
-    // for one more LDS round, with write-through stores of those lines: N = 2^10,
-    // B = 65536 (8 elements): 104 -> 99 us, 2^13, B = 8192 (16): 101 -> 97; at
-    // cores of 2^14 and 2^15 points the one or two blocks of a CU wait longer in
-    // the round than they gain (2^16, B = 1000: 136 -> 143).  The same for the
-    // C2R bins on the way in, with 32 elements, took 10% more at N = 2^13 up to B
-    // = 512 and 3% more past the caches, and 2-4% more at 2^14.
-    constexpr bool BINS_OUT = MODE == 1 && C::PAIR && LOGL <= 13;
+    static_assert(!LINES || (MODE == 1 && C::PAIR && C::TPB * (L + 1) <= C::LDS_FLOATS / (C::SPLIT ? 1 : 2)),
+                  "whole-line bin stores: a lane-paired r2c kernel whose bins fit its LDS rows");
     static_assert(!(C::SPLIT && MODE == 1 && C::LE != 5 && !C::PAIR),
                   "16-element r2c kernels without lane pairing stitch whole complex values out of LDS");
     __shared__ float2 lds_raw[NEED_LDS ? (C::LDS_FLOATS + 1) / 2 : 1];
@@ -448,40 +445,47 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
         // r2c under lane pairing: v[q] = Z[j + T*q] and the mirror of
         // Z[j + T*q] is the partner lane's v[E-1-q] (own v[E-1-q] for
         // j = T/2, own v[(E-q) mod E] for j = 0), so every bin is stitched
-        // in registers and stored once; thread j = 0 also has bin L.  A
-        // transform spans whole waves, and the threads of rows past the batch
-        // hold its last row: every lane swap runs with all lanes of the wave.
+        // in registers and stored once; thread j = 0 also has bin L.
         static_assert(C::logr(P - 1) == C::LE, "lane pairing needs a full radix last pass");
         const bool jz = j == 0, jh = j == T / 2;
-        const float2 tj = tw_real[j];  // tw_real[j + T*s] = tj * exp(-2 pi i s / 2E)
-        const float2 ny = r2c_bin(v[0], v[0], tw_real[L], scale, true);  // bin L, kept by j = 0
-        float2 prev = v[0];  // Z of element (E - s) mod E, which an earlier pair may have turned into a bin
-        float2* const xo = (float2*)dst_v + row * (L + 1) + j;
-        static_for<0, E / 2>([&](auto ss) {
-            constexpr int s = ss.value;
-            constexpr int sb = E - 1 - s;
-            const float2 a = v[s], b = v[sb];
-            const float2 pa = swap_halves(b), pb = swap_halves(a);
-            const float2 ma = jz ? prev : (jh ? b : pa);
-            const float2 mb = jz ? v[s + 1] : (jh ? a : pb);
-            const float2 xa = r2c_bin(a, ma, rot<2 * E, s, -1>(tj), scale, s == 0 && jz);
-            const float2 xb = r2c_bin(b, mb, rot<2 * E, sb, -1>(tj), scale, false);
-            prev = b;
-            if constexpr (BINS_OUT) {
-                v[s] = xa;
-                v[sb] = xb;
+        // put(element, its bin) for the bins of this thread, a pair at a time;
+        // tw_real[j + T*s] = tj * exp(-2 pi i s / 2E).  `prev`: Z of element
+        // (E - s) mod E where put overwrites it (LINES).
+        auto stitch = [&](auto&& put) {
+            const float2 tj = tw_real[j];
+            float2 prev = v[0];
+            static_for<0, E / 2>([&](auto ss) {
+                constexpr int s = ss.value;
+                constexpr int sb = E - 1 - s;
+                const float2 a = v[s], b = v[sb];
+                const float2 pa = swap_halves(b), pb = swap_halves(a);
+                const float2 ma = jz ? (LINES ? prev : v[(E - s) % E]) : (jh ? b : pa);
+                const float2 mb = jz ? v[s + 1] : (jh ? a : pb);
+                prev = b;
+                put(ic<s>{}, r2c_bin(a, ma, rot<2 * E, s, -1>(tj), scale, s == 0 && jz));
+                put(ic<sb>{}, r2c_bin(b, mb, rot<2 * E, sb, -1>(tj), scale, false));
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        if constexpr (!LINES) {
+            // A transform spans whole waves, so `active` is wave-uniform and the
+            // lane swaps run with every lane of the wave or none.
+            if (active) {
+                float2* xo = (float2*)dst_v + row * (L + 1);
+                stitch([&](auto q, float2 x) { xo[j + q.value * T] = x; });
+                if (jz) xo[L] = r2c_bin(v[0], v[0], tw_real[L], scale, true);
+            }
+        } else {
+            // Out through LDS: element e of the block's TPB * (L + 1) bins goes
+            // to lane (e + sh) mod 64, so a store instruction writes whole lines
+            // but for the block's first and last, which its neighbours share.
+            const float2 ny = r2c_bin(v[0], v[0], tw_real[L], scale, true);  // bin L, kept by j = 0
+            stitch([&](auto q, float2 x) {
+                v[q.value] = x;
                 // computed here: sunk below the exchange's first barrier, the
                 // imaginary parts would keep every pair's operands in registers
-                asm volatile("" : "+v"(v[s].x), "+v"(v[s].y), "+v"(v[sb].x), "+v"(v[sb].y));
-            } else if (active) {
-                xo[s * T] = xa;
-                xo[sb * T] = xb;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        if constexpr (BINS_OUT) {
-            // out through LDS: element e of the block's TPB * (L + 1) bins goes to
-            // lane (e + sh) mod 64, so every store instruction writes whole lines
+                asm volatile("" : "+v"(v[q.value].x), "+v"(v[q.value].y));
+            });
             const int64_t first = (int64_t)blockIdx.x * C::TPB;
             const int here = C::TPB == 1 || rows - first > C::TPB ? C::TPB : (int)(rows - first);
             float2* const xb = (float2*)dst_v + first * (L + 1);
@@ -519,8 +523,6 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
                     store_out<true>(byte_off(xa + r.value * C::WG, (uint32_t)tid * 8u),
                                     r.value == E ? tail : v[r.value % E]);
             });
-        } else if (active && jz) {
-            xo[L] = ny;
         }
     } else if constexpr (MODE == 1 && C::SPLIT) {
         // r2c with 32 elements per thread and no lane pairing (the last
@@ -638,7 +640,7 @@ struct LdsArgs {
     bool staged;  // C2C of fewer than 16 threads per transform: in and out through LDS
 };
 
-template <int LOGL, int LOGE, int DIR, int MODE, bool STAGED = false>
+template <int LOGL, int LOGE, int DIR, int MODE, bool STAGED = false, bool LINES = false>
 hipError_t launch_one(const LdsArgs& a) {
     using C = LdsCfg<LOGL, LOGE>;
     const int64_t blocks = (a.rows + C::TPB - 1) / C::TPB;
@@ -649,7 +651,7 @@ hipError_t launch_one(const LdsArgs& a) {
         // blocks one wave of the grid holds (occupancy query, once per kernel)
         static const int per_cu = [] {
             int b = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, lds_fft_kernel<LOGL, LOGE, DIR, MODE, STAGED>, C::WG,
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, lds_fft_kernel<LOGL, LOGE, DIR, MODE, STAGED, LINES>, C::WG,
                                                              0) !=
                 hipSuccess) {
                 (void)hipGetLastError();
@@ -661,10 +663,28 @@ hipError_t launch_one(const LdsArgs& a) {
         // only when the launch runs at least two waves of blocks
         if (wave > 0 && blocks >= 2 * wave) wave_blocks = (int)wave, n = a.stagger;
     }
-    lds_fft_kernel<LOGL, LOGE, DIR, MODE, STAGED><<<(unsigned)blocks, C::WG, 0, a.stream>>>(
+    lds_fft_kernel<LOGL, LOGE, DIR, MODE, STAGED, LINES><<<(unsigned)blocks, C::WG, 0, a.stream>>>(
         a.src, a.dst, a.tw, a.tw_real, a.rows, a.scale, wave_blocks, a.num_cus / 8, n);
     mark(a.stream);
     return hipGetLastError();
+}
+
+// R2C: whole-line bin stores (LINES) from 2^22 samples a launch, where samples
+// and bins (32 MiB) no longer fit the eight 4 MiB L2s, which till then merge the
+// partial lines by themselves; a smaller launch only pays the LDS round (N =
+// 2^10, B = 64: 3.3 us against 3.7, 2^12, B = 256: 5.4 against 5.8).  From there
+// N = 2^10, B = 4096: 8.46 -> 6.97 us, B = 65536: 99.9 -> 91.7; 2^12, B = 1024:
+// 9.84 -> 8.21, B = 16384: 107 -> 101; 2^13, B = 512: 9.98 -> 8.18, B = 8192: 105
+// -> 102.  Not at cores of 2^13 points and more, whose one or two blocks a CU
+// wait longer in the round than they gain (N = 2^14, B = 2048: 55.3 -> 58.8 us,
+// B = 8192: 217 -> 222; 2^16, B = 1000: 136 -> 143), and not with 32 elements,
+// whose two forms round differently: the bits of a row would depend on the batch.
+template <int LOGL, int LOGE>
+hipError_t launch_r2c(const LdsArgs& a) {
+    if constexpr (LOGL <= 12 && LOGE <= 4 && LdsCfg<LOGL, LOGE, 1>::PAIR) {
+        if (a.rows << (LOGL + 1) >= (int64_t)1 << 22) return launch_one<LOGL, LOGE, -1, 1, false, true>(a);
+    }
+    return launch_one<LOGL, LOGE, -1, 1>(a);
 }
 
 template <int LOGL, int LOGE>
@@ -679,7 +699,7 @@ hipError_t dispatch_mode(int mode, int dir, const LdsArgs& a) {
     }
     if (a.staged) return hipErrorInvalidValue;  // refused at plan creation
     if (mode == 0) return dir < 0 ? launch_one<LOGL, LOGE, -1, 0>(a) : launch_one<LOGL, LOGE, 1, 0>(a);
-    if (mode == 1) return launch_one<LOGL, LOGE, -1, 1>(a);
+    if (mode == 1) return launch_r2c<LOGL, LOGE>(a);
     return launch_one<LOGL, LOGE, 1, 2>(a);
 }
 

@@ -274,8 +274,9 @@ __device__ __forceinline__ void store_nt(float2* p, float2 x) {
 // waits for.  Measured in the benchmark's cycle of sizes: the C2C LDS
 // kernel 3-4% faster per launch up to 2^13 points (2-3% slower at 2^14 and
 // 2^15, which keep plain stores) and each four-step pass 1-3% faster.  Rows
-// that are not line-aligned (R2C's bins) keep plain stores: partial lines
-// written through cost more than they save.
+// that are not line-aligned (R2C's bins) keep plain stores, as partial lines
+// written through cost more than they save, unless they go out through LDS in
+// whole lines.
 template <bool WT>
 __device__ __forceinline__ void store_out(float2* p, float2 x) {
     if constexpr (WT)

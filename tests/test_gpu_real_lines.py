@@ -1,6 +1,7 @@
 """Bin rows of n/2 + 1 values, which start anywhere in a 128-byte line, in the
-real modes of the LDS kernel: several rows a block, a ragged last block and
-nothing written outside the rows, against 64-bit numpy.
+real modes of the LDS kernel: several rows a block, a ragged last block, bins
+stored straight or in whole lines, and nothing written outside the rows,
+against 64-bit numpy.
 
 The bound is that of the transform's own rounding: below u per radix-2 level
 and for the stitch (u = 2^-24), so u sqrt(log2 n + 2) in the 2-norm; a bin in
@@ -91,3 +92,36 @@ def test_default_kernel_is_the_same_at_every_batch(gpu, logn, kind):
         elems.append(plan.info.elems_per_thread)
     assert elems[0] == elems[1], elems
     assert torch.equal(rows[0], rows[1])
+
+
+# the lane-paired r2c kernels that store whole lines in launches of 2^22 samples or more
+LINE_CASES = [(10, 8), (11, 16), (12, 16), (13, 8), (13, 16)]
+
+
+@pytest.mark.parametrize("extra,shift", [(-1, 0), (0, 1), (3, 15)])
+@pytest.mark.parametrize("logn,elems", LINE_CASES)
+def test_bin_rows_of_a_large_launch(gpu, logn, elems, extra, shift):
+    """One row below the launch size from which bins go out in whole lines, at
+    it, and a ragged batch above it; the rows have the bits of a small launch."""
+    import torch
+
+    n, m = 1 << logn, (1 << (logn - 1)) + 1
+    batch = (1 << (22 - logn)) + extra
+    x = np.random.default_rng(100 * logn + elems).standard_normal((batch, n)).astype(np.float32)
+    stream = torch.cuda.current_stream().cuda_stream
+    xin = torch.from_numpy(x).to(gpu)
+    first = GUARD + shift
+    buf = torch.full((first + batch * m + GUARD,), 7.0 + 5.0j, dtype=torch.complex64, device=gpu)
+    plan = _plan(n, batch, "r2c", elems)
+    plan.execute(xin.data_ptr(), buf[first:].data_ptr(), stream)
+    small = torch.empty((2, m), dtype=torch.complex64, device=gpu)
+    plan2 = _plan(n, 2, "r2c", elems)
+    plan2.execute(xin[batch - 2:].data_ptr(), small.data_ptr(), stream)
+    torch.cuda.synchronize()
+    got = buf.cpu().numpy()
+    assert np.all(got[:first] == 7 + 5j) and np.all(got[first + batch * m:] == 7 + 5j)
+    got = got[first:first + batch * m].reshape(batch, m)
+    e = np.fft.rfft(x.astype(np.float64), norm="ortho")
+    err = np.linalg.norm(got - e, axis=1) / np.linalg.norm(e, axis=1)
+    assert err.max() <= U * math.sqrt(logn + 2), (int(err.argmax()), float(err.max()))
+    assert np.array_equal(got[batch - 2:].view(np.uint64), small.cpu().numpy().view(np.uint64))
