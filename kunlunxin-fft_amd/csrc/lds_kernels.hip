@@ -154,10 +154,21 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
                   "the staged form is for transforms of fewer than 16 threads");
     // rows of L + 1 bins (R2C output, C2R input) of the staged form, flat in LDS
     static_assert(!STAGED || C::TPB * (L + 1) <= (C::LDS_FLOATS / 2), "staged bin rows exceed the LDS rows");
-    // C2C loads with a select each: at 2^15 points, one 16-wave block per CU,
-    // its exec mask spaces the 32 loads of a thread out (a batch of 1000: 107
-    // us, 109 back to back); the 32-element 1024-point kernel spills without.
-    constexpr bool SELECT = MODE == 0 && C::LE == 5 && (LOGL == 10 || LOGL == 15);
+    // Loads that check their row.  Without the check a kernel has no exec mask
+    // and no moves for it, which saves 2-7% of R2C, of lane-paired C2R and of C2C
+    // with 128 threads or more per transform (C2C N = 2^11, B = 512: 4.90 -> 4.76
+    // us, C2R 2^11, B = 32: 5.28 -> 4.91), 2% of C2C with 8 elements and 16-64
+    // threads (N = 2^7, B = 2^17: 41.9 -> 41.0).  Other C2C kernels gain less in
+    // a full batch than one that fills part of a block loses by loading its last
+    // row again (16 elements, N = 2^5..2^9, B = 3: 7-9%), and unpaired C2R kernels
+    // lose 1-6% throughout.  At 2^15 points, one 16-wave block per CU, the check
+    // is always true, but its masks space the 32 loads of a thread out: N = 2^15,
+    // B = 512, 61.0 us against 63.4, B = 1024 114 against 120; the 32-element
+    // 1024-point kernels and R2C at 2^12 spill without.
+    constexpr bool CHECK =
+        MODE == 0   ? LOGL == 15 || (T < 128 && !(C::LE == 5 && LOGL == 11) && !(C::LE == 3 && T >= 16))
+        : MODE == 1 ? C::LE == 5 && LOGL <= 12
+                    : !C::PAIR && C::TPB > 1;
     constexpr bool NEED_LDS = (P > 1) || (MODE == 1) || STAGED;
     // write-through output stores (store_out) for C2C up to 2^13 points,
     // where every store instruction writes whole 128-byte lines: the staged
@@ -194,13 +205,17 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
     const int j = C::PAIR ? pair_j<T>(tid & (T - 1)) : tid & (T - 1);
     const int64_t row = (int64_t)blockIdx.x * C::TPB + tl;
     const bool active = C::TPB == 1 || row < rows;  // one transform per block: the grid is the batch
-    // the threads of rows past the batch (last block) load its last row again
-    // and store nothing: loads without a select run without exec masks
-    const int64_t lrow = active ? row : rows - 1;
     float2* lt = lds + (NEED_LDS ? tl * C::PITCH : 0);
     float* ltf = ldsf + (NEED_LDS ? tl * C::PITCH : 0);
 
     float2 v[E];
+
+    // threads of rows past the batch (last block): without CHECK they load its
+    // last row again and store nothing
+    const int64_t lrow = (CHECK || active) ? row : rows - 1;
+    auto load_in = [&](const float2* x) {
+        return !CHECK || row < rows ? load_nt(x) : make_float2(0.0f, 0.0f);
+    };
 
     // ---- pass-0 operands straight from HBM
     {
@@ -242,7 +257,7 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             const bool jz = j == 0, jh = j == T / 2;
             float2 xny = make_float2(0.0f, 0.0f);
             const float2* xb = (const float2*)src_v + lrow * (L + 1);
-            static_for<0, E>([&](auto q) { v[q.value] = load_nt(xb + j + q.value * T); });
+            static_for<0, E>([&](auto q) { v[q.value] = load_in(xb + j + q.value * T); });
             if (jz) xny = load_nt(xb + L);
             // exp(-2 pi i (j + T*s) / 2L) = tw_real[j] * exp(-2 pi i s / 2E):
             // one table load and compile-time rotations
@@ -280,14 +295,14 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             // floats): real parts first, kept in px, then imaginary parts,
             // on which the pre-twiddle is applied.  Bin L, the partner of
             // bin 0, is loaded by thread 0, which holds bin 0.
-            const float2* xb = (const float2*)src_v + lrow * (L + 1);
+            const float2* xb = (const float2*)src_v + row * (L + 1);
             static_for<0, NB0>([&](auto m) {
                 static_for<0, R0>([&](auto q) {
                     const int i = j + m.value * T + q.value * (L / R0);
-                    v[m.value * R0 + q.value] = load_nt(xb + i);
+                    v[m.value * R0 + q.value] = load_in(xb + i);
                 });
             });
-            const float2 xny = j == 0 ? load_nt(xb + L) : make_float2(0.0f, 0.0f);
+            const float2 xny = (active && j == 0) ? load_nt(xb + L) : make_float2(0.0f, 0.0f);
             const int pjf = padf<C::FSH>(j);
             float px[E];
             static_for<0, 2>([&](auto comp) {
@@ -325,17 +340,21 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             // transform per 32 lanes (no lane pairing; the partner values
             // would not fit the register budget): both bins straight from
             // global memory
-            const float2* xb = (const float2*)src_v + lrow * (L + 1);
+            const float2* xb = (const float2*)src_v + row * (L + 1);
             static_for<0, NB0>([&](auto m) {
                 static_for<0, R0>([&](auto q) {
                     const int i = j + m.value * T + q.value * (L / R0);
-                    float2 xk = xb[i];
-                    float2 xj = xb[L - i];
-                    if (i == 0) {
-                        xk.y = 0.0f;
-                        xj.y = 0.0f;
+                    float2 z = make_float2(0.0f, 0.0f);
+                    if (active) {
+                        float2 xk = xb[i];
+                        float2 xj = xb[L - i];
+                        if (i == 0) {
+                            xk.y = 0.0f;
+                            xj.y = 0.0f;
+                        }
+                        z = c2r_pre_bin(xk, xj, tw_real[i]);
                     }
-                    v[m.value * R0 + q.value] = c2r_pre_bin(xk, xj, tw_real[i]);
+                    v[m.value * R0 + q.value] = z;
                 });
             });
         } else if constexpr (STAGED) {
@@ -362,9 +381,7 @@ __global__ __launch_bounds__((LdsCfg<LOGL, LOGE, MODE>::WG), (LdsCfg<LOGL, LOGE,
             static_for<0, NB0>([&](auto m) {
                 static_for<0, R0>([&](auto q) {
                     const int i = j + m.value * T + q.value * (L / R0);
-                    float2& x = v[m.value * R0 + q.value];
-                    if constexpr (SELECT) x = row < rows ? load_nt(src + i) : make_float2(0.0f, 0.0f);
-                    else x = load_nt(src + i);
+                    v[m.value * R0 + q.value] = load_in(src + i);
                 });
             });
         }
