@@ -149,10 +149,6 @@ __device__ __forceinline__ int opaque(int x) {
     asm volatile("" : "+v"(x));
     return x;
 }
-__device__ __forceinline__ float2 opaque(float2 x) {
-    asm volatile("" : "+v"(x.x), "+v"(x.y));
-    return x;
-}
 
 // Roots of one pass's butterfly b (dft_dit's r: r[i] = w^(2^i)).  KIND 0, a
 // plain column FFT: w = W_(NS R)^k, k = b mod NS, from the pass table tw.
@@ -629,41 +625,17 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG)) void fourstep_c2r_p
     col_store<C, 0, 2>(v, dst + (row << logn), lds, tid, c, j, log_s, 1.0f, g);
 }
 
-// The pass-2 roots of one thread (PassRoots, KIND 1) held in registers: its
-// column and its butterflies do not change from group to group.
-template <class C, int KIND>
-struct HeldRoots {
-    static constexpr int first(int p) {  // roots of the passes before p
-        int n = 0;
-        for (int q = 0; q < p; ++q) n += (C::E >> C::logr(q)) * C::logr(q);
-        return n;
-    }
-    float2 w[KIND == 1 ? first(C::P) : 1];
-    __device__ __forceinline__ void fill(const PassRoots<C, 1>& from, int j) {
-        static_for<0, C::P>([&](auto p) {
-            constexpr int LR = C::logr(p.value);
-            static_for<0, (C::E >> LR)>([&](auto m) {
-                float2 r[LR];
-                from.template load<p.value, m.value>(r, j + m.value * C::T);
-                static_for<0, LR>([&](auto i) { w[first(p.value) + m.value * LR + i.value] = r[i.value]; });
-            });
-        });
-    }
-    template <int p, int m, int NR>
-    __device__ __forceinline__ void load(float2 (&r)[NR], int) const {
-        constexpr int LR = C::logr(p);
-        static_for<0, LR>([&](auto i) { r[i.value] = opaque(w[first(p) + m * LR + i.value]); });
-    }
-};
-
 // Persistent form of the same pass: gridDim.x blocks, a multiple of the
 // column groups per transform, walk the `tiles` column groups of the launch
-// with stride gridDim.x, so a block keeps one column index c0 (and its
-// four-step twiddles, loaded once) while the batch row advances.  While a
-// group is transformed the next one is already loading into registers, so
-// HBM traffic continues through the block's compute and LDS phases; the pass
-// twiddles sit in LDS, which keeps the only global loads in flight during
-// the compute those of the next group.
+// with stride gridDim.x, so a block keeps one column index c0 while the batch
+// row advances.  While a group is transformed the next one is already loading
+// into registers, so HBM traffic continues through the block's compute and LDS
+// phases; the pass twiddle table and, for pass 2, the W_N^(2^t k1) of the
+// block's columns sit in LDS, which keeps the only global loads in flight during
+// the compute those of the next group.  (Pass 2's roots held in registers across
+// the loop instead spilled 224-240 bytes a lane against 144-160 at 512 and 1024
+// points and took up to 9% more past 2^24 points: N = 2^17, B = 256, n1 = 256: 296
+// us against 264, 2^18, B = 32: 52.4 against 48.0.)
 template <int LOGL, int LOGE, int LOGC, int DIR, int KIND>
 __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG), 4) void fourstep_persist_kernel(
     const float2* src, float2* dst, const float2* __restrict__ tw,
@@ -671,6 +643,7 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG), 4) void fourstep_pe
     using C = ColCfg<LOGL, LOGE, LOGC>;
     __shared__ float2 lds[C::LDS_FLOAT2];
     __shared__ float2 lds_tw[C::TW_SIZE > 0 ? C::TW_SIZE : 1];
+    __shared__ float2 lds_col[KIND == 1 ? LOGL * C::C : 1];  // [t][column]: W_N^(2^t k1)
     const int tid = threadIdx.x;
     const int c = tid & (C::C - 1);
     const int j = tid >> LOGC;
@@ -682,29 +655,25 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG), 4) void fourstep_pe
     const int64_t last_row = (tiles >> log_groups) - 1;
     auto row_of = [&](int64_t t) { return (KIND == 1 && rev) ? last_row - (t >> log_groups) : (t >> log_groups); };
 
-    if constexpr (KIND == 0) {
-        for (int i = tid; i < C::TW_SIZE; i += C::WG) lds_tw[i] = tw[i];
+    for (int i = tid; i < C::TW_SIZE; i += C::WG) lds_tw[i] = tw[i];
+    if constexpr (KIND == 1) {
+        for (int i = tid; i < LOGL * C::C; i += C::WG)
+            lds_col[i] = tw_col[((i >> LOGC) << log_s) + c0 + (i & (C::C - 1))];
     }
-    HeldRoots<C, KIND> held;
-    if constexpr (KIND == 1) held.fill(PassRoots<C, 1>{tw, tw_col + c0 + c, log_s}, j);
     float2 v[C::E];
     col_load<C>(v, src + (row_of(t0) << logn) + c0, c, j, log_s);
-    __syncthreads();  // lds_tw complete
+    __syncthreads();  // lds_tw, lds_col complete
 
     // one column group: transform v (group t) and store it.  Per-call copies
-    // of the loop invariants: recomputing addresses and the pass and
-    // four-step twiddles costs less than the registers that holding them
-    // across the loop (next to the prefetched group) would take.
+    // of the loop invariants: recomputing addresses and roots costs less than the
+    // registers that holding them across the loop (next to the prefetched
+    // group) would take.
     auto process = [&](int64_t t) {
         const int jl = opaque(j), cl = opaque(c), tl = opaque(tid);
-        if constexpr (KIND == 1) {
-            float2 r0[C::LOG_E];
-            held.template load<0, 0>(r0, jl);
-            col_passes<C, DIR, 1, true>(v, lds, cl, jl, r0, held);
-        } else {
-            const float2 r0[C::LOG_E] = {};  // pass 0 has no roots
-            col_passes<C, DIR, 0, true>(v, lds, cl, jl, r0, PassRoots<C, 0>{lds_tw, nullptr, 0});
-        }
+        const PassRoots<C, KIND> roots{lds_tw, KIND == 1 ? lds_col + cl : nullptr, LOGC};
+        float2 r0[C::LOG_E] = {};  // pass 1's pass 0 has no roots
+        if constexpr (KIND == 1) roots.template load<0, 0>(r0, jl);
+        col_passes<C, DIR, KIND, true>(v, lds, cl, jl, r0, roots);
         const int64_t base = row_of(t) << logn;
         col_store<C, KIND>(v, dst + opaque_uniform(KIND == 0 ? base + ((int64_t)c0 << LOGL) : base + c0), lds, tl, cl,
                            jl, log_s, scale);
