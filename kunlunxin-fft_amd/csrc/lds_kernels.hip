@@ -32,8 +32,8 @@
 //      (16 or 32 elements per thread and whole waves per transform: in
 //      registers across lane pairs, the remainder radix running first; 32
 //      elements and 32 lanes per transform: through the output row) and
-//      writes the n/2+1 bins with the scale (lane-paired, core up to 2^12, a
-//      launch past the L2s: through LDS, in whole 128-byte lines)
+//      writes the n/2+1 bins with the scale (lane-paired, core up to 2^13, a
+//      launch past the caches: through LDS, in whole 128-byte lines)
 //   2  c2r: the pre-twiddle of kernels.py:1180-1229 is applied while loading
 //      the n/2+1 bins; the inverse core writes the n real samples as n/2
 //      complex pairs with scale 2*norm_scale
@@ -686,20 +686,29 @@ hipError_t launch_one(const LdsArgs& a) {
     return hipGetLastError();
 }
 
-// R2C: whole-line bin stores (LINES) from 2^22 samples a launch, where samples
-// and bins (32 MiB) no longer fit the eight 4 MiB L2s, which till then merge the
-// partial lines by themselves; a smaller launch only pays the LDS round (N =
-// 2^10, B = 64: 3.3 us against 3.7, 2^12, B = 256: 5.4 against 5.8).  From there
-// N = 2^10, B = 4096: 8.46 -> 6.97 us, B = 65536: 99.9 -> 91.7; 2^12, B = 1024:
-// 9.84 -> 8.21, B = 16384: 107 -> 101; 2^13, B = 512: 9.98 -> 8.18, B = 8192: 105
-// -> 102.  Not at cores of 2^13 points and more, whose one or two blocks a CU
-// wait longer in the round than they gain (N = 2^14, B = 2048: 55.3 -> 58.8 us,
-// B = 8192: 217 -> 222; 2^16, B = 1000: 136 -> 143), and not with 32 elements,
-// whose two forms round differently: the bits of a row would depend on the batch.
+// R2C: whole-line bin stores (LINES) in launches of at least this many samples.
+// Cores up to 2^12: from 2^22, where samples and bins (32 MiB) no longer fit the
+// eight 4 MiB L2s, which till then merge the partial lines by themselves; a
+// smaller launch only pays the LDS round (N = 2^10, B = 64: 3.3 us against 3.7,
+// 2^12, B = 256: 5.4 against 5.8).  From there N = 2^10, B = 4096: 8.46 -> 6.97
+// us, B = 65536: 99.9 -> 91.7; 2^12, B = 1024: 9.84 -> 8.21, B = 16384: 107 ->
+// 101; 2^13, B = 512: 9.98 -> 8.18, B = 8192: 105 -> 102 (N = 2^11 and 2^12 at
+// 2^25 samples lose 2%: 48.2 -> 49.4).  Core 2^13, whose two blocks a CU wait
+// longer in the round: past 2^25, where samples and bins leave the 256 MiB MALL
+// (N = 2^14, B = 2048: 55.6 us against 56.9, B = 3000: 83.8 -> 82.4, B = 4096: 110
+// -> 109).  Longer cores, one block a CU, lose (2^16, B = 1000: 136 -> 143).  Not
+// with 32 elements, whose two forms round differently: the bits of a row would
+// depend on the batch.
+constexpr int64_t kNoLines = INT64_MAX;
+constexpr int64_t lines_from(int logl, int loge) {
+    if (loge > 4 || logl > 13) return kNoLines;
+    return logl <= 12 ? (int64_t)1 << 22 : ((int64_t)1 << 25) + 1;
+}
+
 template <int LOGL, int LOGE>
 hipError_t launch_r2c(const LdsArgs& a) {
-    if constexpr (LOGL <= 12 && LOGE <= 4 && LdsCfg<LOGL, LOGE, 1>::PAIR) {
-        if (a.rows << (LOGL + 1) >= (int64_t)1 << 22) return launch_one<LOGL, LOGE, -1, 1, false, true>(a);
+    if constexpr (LdsCfg<LOGL, LOGE, 1>::PAIR && lines_from(LOGL, LOGE) < kNoLines) {
+        if (a.rows << (LOGL + 1) >= lines_from(LOGL, LOGE)) return launch_one<LOGL, LOGE, -1, 1, false, true>(a);
     }
     return launch_one<LOGL, LOGE, -1, 1>(a);
 }

@@ -94,34 +94,39 @@ def test_default_kernel_is_the_same_at_every_batch(gpu, logn, kind):
     assert torch.equal(rows[0], rows[1])
 
 
-# the lane-paired r2c kernels that store whole lines in launches of 2^22 samples or more
-LINE_CASES = [(10, 8), (11, 16), (12, 16), (13, 8), (13, 16)]
+# the lane-paired r2c kernels that store whole lines in large launches, and the
+# first batch that does: 2^22 samples, past 2^25 at a core of 2^13
+LINE_CASES = [(10, 8, 4096), (11, 16, 2048), (12, 16, 1024), (13, 8, 512), (13, 16, 512), (14, 16, 2049)]
 
 
 @pytest.mark.parametrize("extra,shift", [(-1, 0), (0, 1), (3, 15)])
-@pytest.mark.parametrize("logn,elems", LINE_CASES)
-def test_bin_rows_of_a_large_launch(gpu, logn, elems, extra, shift):
+@pytest.mark.parametrize("logn,elems,first_batch", LINE_CASES)
+def test_bin_rows_of_a_large_launch(gpu, logn, elems, first_batch, extra, shift):
     """One row below the launch size from which bins go out in whole lines, at
-    it, and a ragged batch above it; the rows have the bits of a small launch."""
+    it, and a ragged batch above it: every row has the bits that small launches
+    give, and those of the edges and some between are right."""
     import torch
 
     n, m = 1 << logn, (1 << (logn - 1)) + 1
-    batch = (1 << (22 - logn)) + extra
-    x = np.random.default_rng(100 * logn + elems).standard_normal((batch, n)).astype(np.float32)
+    batch = first_batch + extra
     stream = torch.cuda.current_stream().cuda_stream
-    xin = torch.from_numpy(x).to(gpu)
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(100 * logn + elems)
+    x = torch.randn((batch, n), device=gpu, generator=gen)
     first = GUARD + shift
     buf = torch.full((first + batch * m + GUARD,), 7.0 + 5.0j, dtype=torch.complex64, device=gpu)
-    plan = _plan(n, batch, "r2c", elems)
-    plan.execute(xin.data_ptr(), buf[first:].data_ptr(), stream)
-    small = torch.empty((2, m), dtype=torch.complex64, device=gpu)
-    plan2 = _plan(n, 2, "r2c", elems)
-    plan2.execute(xin[batch - 2:].data_ptr(), small.data_ptr(), stream)
+    large = _plan(n, batch, "r2c", elems)
+    large.execute(x.data_ptr(), buf[first:].data_ptr(), stream)
+    small = torch.empty((batch, m), dtype=torch.complex64, device=gpu)
+    plans = []
+    for r in range(0, batch, 256):
+        plans.append(_plan(n, min(256, batch - r), "r2c", elems))
+        plans[-1].execute(x[r:].data_ptr(), small[r:].data_ptr(), stream)
     torch.cuda.synchronize()
-    got = buf.cpu().numpy()
-    assert np.all(got[:first] == 7 + 5j) and np.all(got[first + batch * m:] == 7 + 5j)
-    got = got[first:first + batch * m].reshape(batch, m)
-    e = np.fft.rfft(x.astype(np.float64), norm="ortho")
-    err = np.linalg.norm(got - e, axis=1) / np.linalg.norm(e, axis=1)
-    assert err.max() <= U * math.sqrt(logn + 2), (int(err.argmax()), float(err.max()))
-    assert np.array_equal(got[batch - 2:].view(np.uint64), small.cpu().numpy().view(np.uint64))
+    got = buf[first:first + batch * m].view(batch, m)
+    assert torch.equal(torch.view_as_real(got), torch.view_as_real(small))
+    assert torch.all(buf[:first] == 7 + 5j) and torch.all(buf[first + batch * m:] == 7 + 5j)
+    rows = [0, 1, 2, 3, 4, batch // 3, batch // 2, batch - 5, batch - 4, batch - 3, batch - 2, batch - 1]
+    e = np.fft.rfft(x[rows].cpu().numpy().astype(np.float64), norm="ortho")
+    y = got[rows].cpu().numpy()
+    assert np.all(np.linalg.norm(y - e, axis=1) <= U * math.sqrt(logn + 2) * np.linalg.norm(e, axis=1))
