@@ -2,11 +2,12 @@
 passes that a transform is cut into, against 64-bit numpy.
 
 The bound is on the rounding of the network itself.  A radix-2 level writes
-each value after two roundings of at most half an ulp (three where the second
-output is derived from the first), whose errors, u = 2^-24, have a variance of
-u^2/3 relative to the value; with the rounding of the roots a level adds less
-than u^2, so log2 N levels stay below u sqrt(log2 N) in the 2-norm.  A wrong
-or misplaced root gives an error of order one.
+each value after two roundings of at most half an ulp (three where the product
+with the root is rounded first, two of them on the smaller product), whose
+errors, u = 2^-24, have a variance of u^2/3 relative to the value; with the
+rounding of the roots a level adds less than u^2, so log2 N levels stay below
+u sqrt(log2 N) in the 2-norm.  A wrong or misplaced root gives an error of order
+one.
 """
 import math
 
@@ -36,7 +37,8 @@ def _run(pkg, gpu, n, batch, direction, executed, params, seed):
 @pytest.mark.parametrize("l1,l2", [(4, 4), (5, 4), (4, 6), (6, 5), (7, 6), (8, 7), (7, 9), (9, 8), (10, 8), (10, 10)])
 def test_four_step_split(pkg, gpu, l1, l2, schedule, direction):
     """Pass 2's roots carry W_N^(n2 k1): every pass length 16..1024 on either
-    side, so every radix 2..32 as first, middle and remainder pass."""
+    side, which takes first radices 4 to 32, middle radices 4 to 16 and last
+    radices 2 to 32."""
     n = 1 << (l1 + l2)
     err = _run(pkg, gpu, n, 3, direction, "fft_four_step_batch", {"n1": 1 << l1, "schedule": schedule},
                1000 * l1 + l2)
@@ -70,31 +72,42 @@ def test_lds_32_elements(pkg, gpu, logn, direction):
     assert err <= U * math.sqrt(logn), err
 
 
-@pytest.mark.parametrize("logn", [4, 5, 6, 7, 8, 10, 11])
+@pytest.mark.parametrize("logn", [4, 5, 6, 7, 8, 9, 10, 11])
 @pytest.mark.parametrize("batch", [1, 3, 257])
-def test_lds_last_block_rows(pkg, gpu, logn, batch):
+def test_lds_last_block_rows(gpu, logn, batch):
     """Several transforms a block: the threads of rows past the batch load its
-    last row again and store nothing, in each mode."""
+    last row again, or nothing, and store nothing, in each mode with every
+    element count it takes."""
     import torch
 
-    n = 1 << logn
+    from kunlunxin_fft_amd import native
+
+    n, m = 1 << logn, (1 << (logn - 1)) + 1
     x = np.random.default_rng(n + batch).standard_normal((batch, n)).astype(np.float32)
-    xin = torch.from_numpy(x[0] if batch == 1 else x).to(gpu)
+    e = np.fft.fft(x.astype(np.float64), norm="ortho")
+    tol = U * math.sqrt(2 * (logn + 2))
+    xin = torch.from_numpy(x).to(gpu)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(kind, elems, src, out):
+        plan = native.NativePlan(n, batch, kind, "inverse" if kind == "c2r" else "forward", norm="ortho",
+                                 flow=native.FLOW_LDS_FUSED, params=[elems])
+        assert plan.info.elems_per_thread == elems
+        plan.execute(src.data_ptr(), out.data_ptr(), stream)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    def close(y, ref):
+        return np.linalg.norm(y - ref) <= tol * np.linalg.norm(ref)
+
     for elems in (4, 8, 16, 32):
-        if elems == 32 and logn < 11:
-            continue
-        common = dict(n=n, batch=batch, direction="dit", precision="fp32", selection_source="table", reason="test",
-                      fallback=False, executed="fft_lds_fused_batch", block=None, params={"elems": elems}, norm="ortho")
-        spec = pkg.execute_fft_plan(pkg.ExecutionPlan(transform_type="r2c", **common), xin)
-        back = pkg.execute_fft_plan(pkg.ExecutionPlan(transform_type="c2r", transform_direction="inverse", **common),
-                                    spec)
-        cplx = pkg.execute_fft_plan(pkg.ExecutionPlan(**common), xin.to(torch.complex64))
-        e = np.fft.fft(x.astype(np.float64), norm="ortho")
-        tol = U * math.sqrt(2 * (logn + 2))
-        assert np.linalg.norm(cplx.cpu().numpy().reshape(batch, -1) - e) <= tol * np.linalg.norm(e)
-        half = e[:, : n // 2 + 1]
-        assert np.linalg.norm(spec.cpu().numpy().reshape(batch, -1) - half) <= tol * np.linalg.norm(half)
-        assert np.linalg.norm(back.cpu().numpy().reshape(batch, -1) - x) <= tol * np.linalg.norm(x)
+        if elems < 32 or logn >= 10:
+            cplx = xin.to(torch.complex64)
+            assert close(run("c2c", elems, cplx, torch.empty_like(cplx)), e), elems
+        if elems < 32 or logn >= 11:  # a real transform's core is n/2
+            spec = torch.empty((batch, m), dtype=torch.complex64, device=gpu)
+            assert close(run("r2c", elems, xin, spec), e[:, :m]), elems
+            assert close(run("c2r", elems, spec, torch.empty_like(xin)), x), elems
 
 
 MAX = float(np.finfo(np.float32).max)
