@@ -5,13 +5,13 @@
 // N = N1*N2, n = n1*N2 + n2, k = k1 + N1*k2:
 //   X[k1 + N1*k2] = sum_n2 W_N2^(n2*k2) * [ W_N^(n2*k1) * sum_n1 x[n1*N2+n2] W_N1^(n1*k1) ]
 // Pass 1 (column pass): for each n2, an N1-point FFT down the column
-//   x[n1*N2 + n2] (row stride N2), times W_N^(n2*k1), stored transposed as
-//   Z[n2*N1 + k1] -- one contiguous run of N1 per column, so the store is
-//   unit-stride.  The twiddle and the layout hand-off are fused into this
-//   store (the reference's k_twiddle_fused idea, issue10_wp3_perf.py:214-242).
-// Pass 2 (row pass): for each k1, an N2-point FFT over Z[k1 + N1*n2] (stride
-//   N1), stored to X[k1 + N1*k2] -- the same addresses it read, so pass 2 runs
-//   in place on the output buffer and the plan needs no workspace.
+//   x[n1*N2 + n2] (row stride N2), stored transposed as Z[n2*N1 + k1] -- one
+//   contiguous run of N1 per column, so the store is unit-stride and the layout
+//   hand-off costs no pass of its own (the reference's k_twiddle_fused idea,
+//   issue10_wp3_perf.py:214-242).
+// Pass 2 (row pass): for each k1, an N2-point FFT over W_N^(n2*k1) Z[k1 + N1*n2]
+//   (stride N1), stored to X[k1 + N1*k2] -- the same addresses it read, so pass 2
+//   runs in place on the output buffer and the plan needs no workspace.
 // Both passes are one kernel template: a block owns C adjacent columns (lanes
 // run along the columns, so every row access is a C*8-byte contiguous run),
 // keeps them in LDS, and runs the same Stockham passes as the single-pass
@@ -393,8 +393,9 @@ __device__ __forceinline__ void col_store(const float2 (&v)[C::E], float2* d, fl
     }
 }
 
-// KIND 0: pass 1 (column FFTs of length L = N1 over S = N2 columns, twiddle,
-//         transposed store).  KIND 1: pass 2 (in place, L = N2, S = N1 columns).
+// KIND 0: pass 1 (column FFTs of length L = N1 over S = N2 columns, transposed
+//         store).  KIND 1: pass 2 (in place, L = N2, S = N1 columns, with the
+//         twiddle in its roots).
 // One column group per block: the C columns [c0, c0 + C) of one batch row.
 // KIND 1 runs in place (src == dst): every element of the block's columns is
 // in registers before the first barrier, all stores come after it, and no
@@ -744,7 +745,8 @@ __global__ __launch_bounds__((ColCfg<LOGL, LOGE, LOGC>::WG), 4) void fourstep_pe
 template <int LL1, int LE1, int LC1, int LL2, int LE2, int LC2, int DIR>
 __global__ __launch_bounds__((ColCfg<LL1, LE1, LC1>::WG)) void fourstep_fused_kernel(
     const float2* src, float2* dst, float2* ring, const float2* __restrict__ tw1, const float2* __restrict__ tw2,
-    const float2* __restrict__ tw_col, float scale, int rows, int nslot, int lag, int nring, int per_take, int* sync, int* overrun, long long wait_ticks) {
+    const float2* __restrict__ tw_col, float scale, int rows, int nslot, int lag, int nring, int per_take, int* sync,
+    int* overrun, long long wait_ticks) {
     using A = ColCfg<LL1, LE1, LC1>;
     using B = ColCfg<LL2, LE2, LC2>;
     static_assert(A::WG == B::WG, "both passes run with the same block size");

@@ -15,7 +15,9 @@
 // owns E = L/T elements (T threads per transform), i.e. E/R butterflies per
 // pass.  Twiddles come from a per-pass table holding, for each span NS, the
 // rows W^(k), W^(2k), W^(4k), W^(8k) (k < NS) -- a few coalesced loads per
-// butterfly; the other powers are composed with one complex product each.
+// butterfly; the other powers are composed with one complex product each, or
+// (32 elements per thread) the loaded ones turn the roots of the DFT's own
+// butterflies (dft_dit).
 // Pass 0 reads HBM directly and the last pass writes HBM directly --
 // both are unit-stride across the lanes of a transform -- and the passes in
 // between exchange through LDS.  With fewer than 16 threads per transform
@@ -668,9 +670,8 @@ hipError_t launch_one(const LdsArgs& a) {
         // blocks one wave of the grid holds (occupancy query, once per kernel)
         static const int per_cu = [] {
             int b = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, lds_fft_kernel<LOGL, LOGE, DIR, MODE, STAGED, LINES>, C::WG,
-                                                             0) !=
-                hipSuccess) {
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                    &b, lds_fft_kernel<LOGL, LOGE, DIR, MODE, STAGED, LINES>, C::WG, 0) != hipSuccess) {
                 (void)hipGetLastError();
                 b = 0;
             }

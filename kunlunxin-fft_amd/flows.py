@@ -58,17 +58,17 @@ def flow_params(executed: str, n: int, transform_type: str, block, params: dict)
             return native.FLOW_AUTO, ()
         if e == 32 and logc < 10:
             e = 0
-        # r2c cores below 32768 run with 16 elements per thread: the
-        # 32-element kernel stitches through the output row (one more pass
-        # over it, measured 1.3-1.8x slower there); at 32768 it is the only
-        # single-pass form
-        if e == 32 and transform_type == "r2c" and logc < 15:
-            e = 16
-        # c2r cores below 32768 run with 16 elements per thread: they load
-        # each bin once and pair it with its mirror bin through LDS, where the
-        # 32-element kernel (no registers to spare for the pairs) loads every
-        # bin twice (measured 1.3-1.5x slower at 2^10-2^14 points)
-        if e == 32 and transform_type == "c2r" and logc < 15:
+        # r2c and c2r cores below 32768 run with 16 elements per thread where an
+        # entry, then one measured on the c2c core, says 32; at 32768 it is the
+        # only single-pass form.  Against 16 elements, 32 take (r2c / c2r) at a
+        # core of 2^10 2.6 / 1.9 times as long in a small batch and 2.0 / 1.5 times
+        # past the caches (bins through the output row, or loaded twice), at 2^11
+        # and 2^12 1.6-1.8 times as long in a small batch, up to 10% longer past the
+        # caches, at 2^13 4 / 3% longer (n = 2^14, batch 256: 12.6 -> 13.2 us), 3%
+        # less past the caches (batch 4096: 112 -> 109), and at 2^14 4-6 / 1-4% less
+        # (n = 2^15, batch 256: 21.3 -> 20.1 us; batch 2048: 117 -> 110): the shipped
+        # table's real entries were measured without them.
+        if e == 32 and transform_type != "c2c" and logc < 15:
             e = 16
         if logc >= 13 and 0 < e < 16:
             e = 0
