@@ -161,7 +161,8 @@ def test_execute_rows_sum_every_launch_of_one_execute():
 
 def test_kernel_names_with_a_boolean_template_argument():
     """The LDS kernel's names carry its staged flag (true / false) as a fifth
-    template argument; the size matching reads it as 1 / 0."""
+    and its whole-line flag as a sixth template argument; the size matching
+    reads them as 1 / 0."""
     import importlib.util
 
     spec = importlib.util.spec_from_file_location("_pmc_summary", SCRIPT)
@@ -175,4 +176,6 @@ def test_kernel_names_with_a_boolean_template_argument():
         ["lds_fft_kernel|N=1024|rows=32768"]
     real = [{"n": 1024, "batch": 32768, "transform": "r2c", "flow": "lds-fused", "split": None}]
     assert mod.real_keys("lds_fft_kernel<9, 4, -1, 1, false>", (512 * 32768) // 16, real) == \
+        ["r2c lds_fft_kernel|N=1024|rows=32768"]
+    assert mod.real_keys("lds_fft_kernel<9, 4, -1, 1, false, true>", (512 * 32768) // 16, real) == \
         ["r2c lds_fft_kernel|N=1024|rows=32768"]
